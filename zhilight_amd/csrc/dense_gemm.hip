@@ -6,12 +6,15 @@
 // chunks.  fp32 accumulation, one rounding to T (the reference's HIGH_PRECISION GEMM mode).  M <= 4 stays on
 // the wave-per-row GEMV (dense_gemv.hip), which streams at 6.5 TB/s.
 //
-// Same tiling as w4_gemm_tiled.hip without the dequant: workgroup = 4 waves = BM x 128 outputs, wave = BM x 32
+// Up to 32 rows (decode batches: the weights are the traffic) k_dense_gemm, more rows (prompt chunks: the matrix pipe is) zl_gemm16.h.
+//
+// k_dense_gemm: the tiling of w4_gemm_tiled.hip without the dequant: workgroup = 4 waves = BM x 128 outputs, wave = BM x 32
 // (two 16-column weight tiles share every activation fragment), K in 128-k chunks; the activation chunk is
 // double-buffered in LDS; weight fragments (lane = row n, 8 consecutive k: 16 B) are loaded straight into
 // the MFMA B registers two chunks ahead (a 16-row x 128-k tile is 16 x 256 contiguous bytes).
 #include <stdlib.h>
 #include "zl_common.h"
+#include "zl_gemm16.h"
 
 namespace {
 
@@ -168,6 +171,32 @@ __global__ __launch_bounds__(256) void k_dense_pack_m(const uint16_t* __restrict
     out[u] = v;
 }
 
+// y = T(alpha * sum + bias), four columns of a row at a time
+template <int DT>
+struct DenseEpi {
+    uint16_t* y;
+    const uint16_t* bias;
+    float alpha;
+    int vec;                                                   // y rows are 8-byte aligned
+    template <int NI, class F>
+    __device__ __forceinline__ void row(int r, int c0, int n, F sum) const {
+        uint16_t* yr = y + (size_t)r * n;
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            const int c = c0 + 16 * j;
+            const g16_f4 v = sum(j);
+            uint16_t o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = ZT<DT>::from_f32(alpha * v[e] + ((bias && c + e < n) ? ZT<DT>::to_f32(bias[c + e]) : 0.f));
+            if (vec && c + 4 <= n) *reinterpret_cast<uint2*>(yr + c) = make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (c + e < n) yr[c + e] = o[e];
+        }
+    }
+};
+
 }  // namespace
 
 extern "C" int64_t zl_dense_m_bytes(int64_t n, int64_t k) {
@@ -215,7 +244,13 @@ extern "C" int zl_gemm_nt(const uint16_t* x, int64_t ldx, const uint16_t* w, con
     p.m = (int)m; p.n = (int)n; p.k = (int)k; p.groups = (int)(k / 128);
     const unsigned gx = (unsigned)((n + kDBN - 1) / kDBN);
     hipStream_t hs = (hipStream_t)s;
-    const int bm = m <= 16 ? 16 : (m <= 32 ? 32 : 64);
+    if (m > 32 && m < (1 << 30) && n < (1 << 30) && g16_takes(x, ldx, w, k, k)) {
+        const Gemm16P g = {x, w, ldx, k, (int)m, (int)n, (int)k, 0, 0, (int)k};
+        const int vec = n % 4 == 0 && ((uintptr_t)y & 7) == 0;
+        if (dtype == ZL_F16) return g16_launch<ZL_F16>(g, DenseEpi<ZL_F16>{y, bias, alpha, vec}, hs);
+        return g16_launch<ZL_BF16>(g, DenseEpi<ZL_BF16>{y, bias, alpha, vec}, hs);
+    }
+    const int bm = m <= 16 ? 16 : 32;                          // (more rows only with row strides that zl_gemm16.h does not take)
     ZL_CHECK_ARG((m + bm - 1) / bm <= 65535, ZL_ELIMIT);
     const dim3 grid(gx, (unsigned)((m + bm - 1) / bm));
 #ifndef ZL_DENSE_NS
@@ -223,8 +258,7 @@ extern "C" int zl_gemm_nt(const uint16_t* x, int64_t ldx, const uint16_t* w, con
 #endif
 #define ZL_DG(DT)                                                                              \
     if (bm == 16) hipLaunchKernelGGL((k_dense_gemm<DT, 16, ZL_DENSE_NS>), grid, dim3(kDT), 0, hs, p);       \
-    else if (bm == 32) hipLaunchKernelGGL((k_dense_gemm<DT, 32, ZL_DENSE_NS>), grid, dim3(kDT), 0, hs, p);  \
-    else hipLaunchKernelGGL((k_dense_gemm<DT, 64>), grid, dim3(kDT), 0, hs, p);
+    else hipLaunchKernelGGL((k_dense_gemm<DT, 32, ZL_DENSE_NS>), grid, dim3(kDT), 0, hs, p);
     if (dtype == ZL_F16) { ZL_DG(ZL_F16) } else { ZL_DG(ZL_BF16) }
 #undef ZL_DG
     return zl_launch_status();

@@ -1,0 +1,185 @@
+// zl_gemm16.h -- the large 16-bit NT product (prompt portions): y (m, n) = x (m, k) . w (n, k)^T on the matrix cores, fp32 accumulation in
+// k order.  One kernel for both libraries: dense_gemm.hip (fp16 / bf16 models) and csrc_seq/seq_gemm.hip (the ragged-step engine).
+//
+// What bounds it: the matrix pipe when an operand tile is large, the latency of its slices when it is small.  Both operands go global -> LDS by
+// LDS-DMA (no registers, no ds_write) into a ring of ST slices of 64 k; a slice is requested ST - 1 slices ahead, there is one barrier per
+// slice, and it sits between the slice's two 32-k halves, so that the second half's MFMAs cover the first LDS reads of the next slice.
+// Measured (bf16, fp32 out, weights cold in HBM): 4096^3 1.06 PFLOP/s; 1024 x 28672 x 4096 1.09; 777 x 6912 x 2304 0.65; 777 x 2304 x 5760
+// 0.57; the kernels it took the place of (64-row tiles with weights straight into registers; 32-k slices through registers and two barriers)
+// ran these at 0.2 .. 0.75.
+#pragma once
+#include "zl_common.h"
+
+typedef _Float16 g16_h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 g16_b8 __attribute__((ext_vector_type(8)));
+typedef float g16_f4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* g16_lds;
+
+struct Gemm16P {
+    const uint16_t* x; const uint16_t* w;
+    int64_t ldx, ldw;                                          // elements
+    int m, n, k;                                               // k % 64 == 0
+    int gx, gy;                                                // tiles along n and m
+    int k_part;                                                // workgroups y = 1, 2, ... take the following k_part numbers of k (whole 64s)
+};
+
+template <int DT>
+__device__ __forceinline__ g16_f4 g16_mfma(uint4 a, uint4 b, g16_f4 c) {
+    if constexpr (DT == ZL_F16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(g16_h8, a), __builtin_bit_cast(g16_h8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(g16_b8, a), __builtin_bit_cast(g16_b8, b), c, 0, 0, 0);
+}
+
+// one LDS-DMA load: 64 lanes x 16 bytes from a descriptor + lane offset + scalar offset to 1 KiB at LDS byte address `lds`.  As asm without
+// outputs: the compiler knows nothing of it, so it neither waits for it nor keeps other LDS reads from running beside it -- the kernel's
+// own waits (g16_wait) order it.
+__device__ __forceinline__ void g16_dma(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %0, %2 offen lds" ::"s"(rsrc), "v"(voff), "s"(soff), "s"(lds) : "m0");
+}
+template <int N>
+__device__ __forceinline__ void g16_wait() {                   // at most N of this wave's loads outstanding, its LDS reads done
+    static_assert(N >= 0 && N < 64, "vmcnt has 6 bits");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ u32x4 g16_rsrc(const void* base) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return (u32x4){(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)), 0xffffffffu, 0x00020000u};
+}
+
+// BM x BN outputs per workgroup of WM x WN waves; slices of 64 numbers of k in a ring of ST LDS buffers.  The weights are the MFMAs' A operand:
+// a lane ends up with four neighbouring columns of one row, which leave in one store.
+template <int DT, int BM, int BN, int WM, int WN, int ST, class Epi>
+__global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm16(const Gemm16P p, const Epi epi) {
+    constexpr int T = 64 * WM * WN, MI = BM / WM / 16, NI = BN / WN / 16, LX = BM * 8 / T, LW = BN * 8 / T;
+    constexpr uint32_t kBuf = (BM + BN) * 128;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char g16_smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nrow = lane & 15, kq = lane >> 4;
+    const int wm = wave % WM, wn = wave / WM;
+    // consecutive workgroups go to the 8 XCDs in turn: an XCD gets a contiguous run of tiles, column by column of 8 row tiles
+    const int total = p.gx * p.gy, q = total >> 3, rem = total & 7, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
+    const int id = xcd * q + min(xcd, rem) + loc;
+    const int band = 8 * p.gx, b = id / band, in = id - b * band, hgt = min(8, p.gy - 8 * b);
+    const int m0 = (8 * b + in % hgt) * BM, n0 = (in / hgt) * BN;
+    const int k0 = blockIdx.y * p.k_part, nt = min(p.k - k0, p.k_part) >> 6;
+    const u32x4 rx = g16_rsrc(p.x + (size_t)m0 * p.ldx + k0), rw = g16_rsrc(p.w + (size_t)n0 * p.ldw + k0);
+    // a wave's load fills 8 LDS rows of 64 k: lane l -> row l / 8, 16-byte unit l % 8, which holds unit (l % 8) ^ (row / 2 % 8) of the
+    // matrix row: a fragment's 16 rows x 16 bytes then lie in 64 different banks.  Rows past the edge read the last row (never stored).
+    uint32_t xo[LX], wo[LW];
+    const int lr = wave * 8 + (lane >> 3), lu = lane & 7;
+#pragma unroll
+    for (int i = 0; i < LX; ++i) {
+        const int r = lr + i * (T / 8);
+        xo[i] = (uint32_t)(min(r, p.m - 1 - m0) * (int)p.ldx * 2 + ((lu ^ ((r >> 1) & 7)) * 16));
+    }
+#pragma unroll
+    for (int i = 0; i < LW; ++i) {
+        const int r = lr + i * (T / 8);
+        wo[i] = (uint32_t)(min(r, p.n - 1 - n0) * (int)p.ldw * 2 + ((lu ^ ((r >> 1) & 7)) * 16));
+    }
+    const uint32_t lds0 = (uint32_t)(size_t)(g16_lds)g16_smem + wave * 1024;
+    auto dma = [&](uint32_t buf, int t) {                      // slice t into the buffer at byte buf
+#pragma unroll
+        for (int i = 0; i < LX; ++i) g16_dma(rx, xo[i], (uint32_t)t * 128, lds0 + buf + i * (T * 16));
+#pragma unroll
+        for (int i = 0; i < LW; ++i) g16_dma(rw, wo[i], (uint32_t)t * 128, lds0 + buf + BM * 128 + i * (T * 16));
+    };
+    const int sw = (nrow >> 1) & 7;
+    const uint32_t fx = (wm * MI * 16 + nrow) * 128, fw = (BM + wn * NI * 16 + nrow) * 128, u0 = (kq ^ sw) * 16, u1 = u0 ^ 64;
+    g16_f4 acc[NI][MI];
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int i = 0; i < MI; ++i) acc[j][i] = (g16_f4){0.f, 0.f, 0.f, 0.f};
+    uint4 fa[2][MI], fb[2][NI];
+    auto rd = [&](int set, uint32_t at) {
+#pragma unroll
+        for (int j = 0; j < NI; ++j) fb[set][j] = *reinterpret_cast<const uint4*>(g16_smem + fw + at + j * 2048);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[set][i] = *reinterpret_cast<const uint4*>(g16_smem + fx + at + i * 2048);
+    };
+    auto mul = [&](int set) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NI; ++j) acc[j][i] = g16_mfma<DT>(fb[set][j], fa[set][i], acc[j][i]);
+    };
+#pragma unroll
+    for (int u = 0; u < ST; ++u)
+        if (u < nt) dma(u * kBuf, u);
+    if (nt >= ST) g16_wait<(ST - 1) * (LX + LW)>();
+    else g16_wait<0>();
+    __builtin_amdgcn_s_barrier();
+    rd(0, u0);
+    uint32_t cur = 0;
+    for (int t = 0; t < nt; ++t) {
+        const uint32_t nxt = cur + kBuf == ST * kBuf ? 0 : cur + kBuf;
+        rd(1, cur + u1);
+        mul(0);
+        // slice t + 1 has landed, every wave holds the rest of slice t in registers: its buffer takes slice t + ST
+        if (t + ST <= nt) g16_wait<(ST - 2) * (LX + LW)>();
+        else g16_wait<0>();
+        __builtin_amdgcn_s_barrier();
+        if (t + ST < nt) dma(cur, t + ST);
+        rd(0, nxt + u0);                                       // (past the last slice: old numbers, never multiplied)
+        mul(1);
+        cur = nxt;
+    }
+    // lane: row nrow of a 16-row block, columns 4 kq .. + 3 of a 16-column block
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int row = m0 + wm * MI * 16 + i * 16 + nrow;
+        if (row < p.m) epi.template row<NI>(row, n0 + wn * NI * 16 + 4 * kq, p.n, [&](int j) { return acc[j][i]; });
+    }
+}
+
+// The tile: the shape whose busiest CU is done first.  `cost` is the measured time of one 64-k slice of one tile (hundredths of a us, cold
+// weights) with the CU as full as the shape's LDS allows, `alone` with one such workgroup per CU; a launch takes ceil(tiles / CUs) of them.  The big
+// tiles win where they come to whole rounds (1024 x 28672: 220 us against 293 with 128 x 128), the deep rings of small tiles where there
+// are fewer tiles than CUs (777 x 2304 x 5760: 36 us with 128 x 64, 77 with 128 x 128 in two slices, 122 with 256 x 256).
+struct Gemm16Tile { int bm, bn, alone, cost; };
+static const Gemm16Tile kGemm16Tiles[6] = {{256, 256, 185, 172}, {256, 128, 100, 100}, {128, 128, 85, 56}, {128, 128, 61, 62}, {128, 64, 42, 40}, {64, 64, 28, 26}};
+
+static inline int g16_pick(int64_t m, int64_t n) {
+    int best = 0;
+    int64_t least = INT64_MAX;
+    for (int i = 0; i < 6; ++i) {
+        const Gemm16Tile& t = kGemm16Tiles[i];
+        const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn), r = (tiles + 255) / 256;
+        const int64_t c = r == 1 ? t.alone : r * t.cost;
+        if (c < least) { least = c; best = i; }
+    }
+    return best;
+}
+
+// whether the kernel takes a product: whole 64-k slices, 16-byte rows, tile offsets that fit 32 bits
+static inline bool g16_takes(const void* x, int64_t ldx, const void* w, int64_t ldw, int64_t k) {
+    return k % 64 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 && ldx <= (1 << 22) && ldw <= (1 << 22);
+}
+
+template <int DT, int BM, int BN, int WM, int WN, int ST, class Epi>
+int g16_launch_tile(Gemm16P p, const Epi& e, hipStream_t s) {
+    const int parts = (p.k + p.k_part - 1) / p.k_part;
+    p.gx = (p.n + BN - 1) / BN;
+    p.gy = (p.m + BM - 1) / BM;
+    if ((int64_t)p.gx * p.gy > INT32_MAX) return ZL_ELIMIT;
+    constexpr int lds = (BM + BN) * 128 * ST;
+    if (lds > 64 * 1024 &&                                     // (every launch: the attribute is per device, one process may drive several)
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm16<DT, BM, BN, WM, WN, ST, Epi>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+        return ZL_ELIMIT;
+    hipLaunchKernelGGL((k_gemm16<DT, BM, BN, WM, WN, ST, Epi>), dim3((unsigned)(p.gx * p.gy), (unsigned)parts), dim3(64 * WM * WN), lds, s, p, e);
+    return zl_launch_status();
+}
+
+template <int DT, class Epi>
+int g16_launch(const Gemm16P& p, const Epi& e, hipStream_t s) {
+    switch (p.k_part < p.k ? 5 : g16_pick(p.m, p.n)) {         // (a divided k: the caller counts 64 x 64 tiles)
+        case 0: return g16_launch_tile<DT, 256, 256, 2, 4, 2>(p, e, s);
+        case 1: return g16_launch_tile<DT, 256, 128, 4, 2, 3>(p, e, s);
+        case 2: return g16_launch_tile<DT, 128, 128, 2, 4, 2>(p, e, s);
+        case 3: return g16_launch_tile<DT, 128, 128, 2, 4, 3>(p, e, s);
+        case 4: return g16_launch_tile<DT, 128, 64, 4, 2, 4>(p, e, s);
+        default: return g16_launch_tile<DT, 64, 64, 2, 2, 4>(p, e, s);
+    }
+}

@@ -9,10 +9,13 @@
 //   k_seq_gemm  more rows (prompt portions, mixed steps): 128 x 128 or 64 x 64 output tile per workgroup of 4 waves (2 x 2; a wave =
 //               4 x 4 or 2 x 2 MFMA tiles of 16 x 16), 32-k slices of x and W staged through LDS (zero-filled past the edges), the next slice's global
 //               loads issued before the current slice's MFMAs.  bf16: v_mfma_f32_16x16x32_bf16; fp32: v_mfma_f32_16x16x4_f32.
+//               bf16 rows whose k comes to whole 64s go to zl_gemm16.h instead (larger tiles through LDS-DMA); this kernel keeps every other
+//               size, fp32, gathered rows and the experts' grouped products.
 //               A long k with few output tiles is divided over workgroups (blockIdx.z), k_split_sum adds the parts.
 // Each has instantiations with an epilogue: EPI 1 adds a bias and writes leading columns once more in the serving format, EPI 2 also applies
 // an activation and a factor looked up per row.
 #include "seq_common.h"
+#include "../csrc/zl_gemm16.h"
 
 namespace {
 
@@ -378,9 +381,68 @@ __global__ __launch_bounds__(256) void k_seq_gemv_grouped(const GemmP p, const i
     if (lane == 0) SeqT<ODT>::st(p.y, (size_t)row * p.ldy + col, a0);
 }
 
+// the results of zl_gemm16.h: four columns of a row at a time through put's steps
+template <int DT, int ODT, int EPI>
+struct SeqEpi {
+    GemmP p;
+    int vec;                                                   // y (and bias) in 16- / 8-byte pieces
+    template <int NI, class F>
+    __device__ __forceinline__ void row(int r, int c0, int n, F sum) const {
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            const int c = c0 + 16 * j;
+            const g16_f4 v = sum(j);
+            if (EPI == 0 && vec && c + 4 <= n) {
+                if constexpr (ODT == ZL_F32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.y) + (size_t)r * p.ldy + c) = make_float4(v[0], v[1], v[2], v[3]);
+                else {
+                    uint32_t o[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[e] = ZT<ZL_BF16>::from_f32(v[e]);
+                    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(p.y) + (size_t)r * p.ldy + c) = make_uint2(o[0] | o[1] << 16, o[2] | o[3] << 16);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (c + e < n) put<DT, ODT, EPI>(p, r, c + e, v[e]);
+            }
+        }
+    }
+};
+
+// the plain sums of a part of k
+struct PartEpi {
+    float* part;
+    int m;
+    template <int NI, class F>
+    __device__ __forceinline__ void row(int r, int c0, int n, F sum) const {
+        float* y = part + ((size_t)blockIdx.y * m + r) * n;
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            const int c = c0 + 16 * j;
+            const g16_f4 v = sum(j);
+            if (n % 4 == 0 && c + 4 <= n) *reinterpret_cast<float4*>(y + c) = make_float4(v[0], v[1], v[2], v[3]);
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (c + e < n) y[c + e] = v[e];
+        }
+    }
+};
+
 // 128 x 128 tiles (four times the MFMAs per LDS fragment) when they still fill the chip, 64 x 64 otherwise
 template <int DT, int ODT, int EPI = 0>
 void launch_tiled(const GemmP& p, hipStream_t hs) {
+    if constexpr (DT == ZL_BF16) {
+        if (!p.x_rows && !p.w_rows && !p.tiles && p.k_part % 64 == 0 && g16_takes(p.x, p.ldx, p.w, p.ldw, p.k)) {
+            const Gemm16P g = {reinterpret_cast<const uint16_t*>(p.x), reinterpret_cast<const uint16_t*>(p.w), p.ldx, p.ldw, p.m, p.n, p.k, 0, 0,
+                               p.part ? p.k_part : p.k};
+            const int vec = p.ldy % 4 == 0 && ((uintptr_t)p.y & 15) == 0;
+            const int rc = p.part ? g16_launch<ZL_BF16>(g, PartEpi{p.part, p.m}, hs) : g16_launch<ZL_BF16>(g, SeqEpi<DT, ODT, EPI>{p, vec}, hs);
+            if (rc == ZL_OK && p.part)
+                hipLaunchKernelGGL((k_split_sum<DT, ODT, EPI>), dim3((unsigned)(((int64_t)p.m * p.n + 255) / 256)), dim3(256), 0, hs, p);
+            if (rc == ZL_OK) return;
+        }
+    }
     const int64_t big = (int64_t)((p.m + 127) / 128) * ((p.n + 127) / 128);
     if (p.part) {
         const dim3 grid((unsigned)((p.n + 63) / 64), (unsigned)((p.m + 63) / 64), (unsigned)p.n_parts);
@@ -431,7 +493,8 @@ extern "C" int zls_gemm_nt_act(const void* x, int64_t ldx, const void* w, const 
     p.x_rows = p.w_rows = nullptr; p.tiles = nullptr; p.w_stride = 0;
     if (part) {
         ZL_CHECK_ARG(n_parts > 0 && n_parts <= 65535, ZL_EINVAL);
-        p.k_part = (int)((k + n_parts * kBK - 1) / (n_parts * kBK) * kBK);
+        const int64_t unit_k = dtype == ZL_BF16 && k % 64 == 0 ? 64 : kBK;                       // (whole slices of the kernel that takes it)
+        p.k_part = (int)((k + n_parts * unit_k - 1) / (n_parts * unit_k) * unit_k);
         p.n_parts = (int)((k + p.k_part - 1) / p.k_part);                // (never more than the caller made room for)
         p.part = part;
     }
