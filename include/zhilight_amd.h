@@ -659,6 +659,10 @@ int zl_prefill_attn(const uint16_t* q, const uint16_t* k_buf, const uint16_t* v_
 int zl_prefill_attn_ex(const uint16_t* q, const uint16_t* k_buf, const uint16_t* v_buf, uint16_t* out, int64_t s_q,
                        int64_t pos0, int64_t h, int64_t hkv, int64_t d, float scale, int64_t len_buf, int bshd,
                        int dtype, int groups, zl_stream_t s);
+/* the same for heads of 64 numbers; the probabilities keep 32-bit quality (two numbers of T each), as in the mask form of zl_decode_attn
+ * (q, k_buf, v_buf 16-byte aligned) */
+int zl_prefill_attn_w32(const uint16_t* q, const uint16_t* k_buf, const uint16_t* v_buf, uint16_t* out, int64_t s_q, int64_t pos0,
+                        int64_t h, int64_t hkv, int64_t d, float scale, int64_t len_buf, int bshd, int dtype, zl_stream_t s);
 
 
 /* ------------------------------------------------------------------------------------------------

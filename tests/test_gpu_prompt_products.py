@@ -69,3 +69,44 @@ def test_a_row_that_is_not_finite_stays_alone():
     for y in (ops.gemm_nt(x, w), seqops.gemm_nt(x, w)):
         rows = torch.isfinite(y).all(1)
         assert not rows[199] and not rows[64] and int(rows.sum()) == 198
+
+
+# ---- prompt attention of 64-wide heads (csrc/prefill_attn.hip, zl_prefill_attn_w32) -----------------------------------------------------
+def _attention64(q, k, v, pos0, scale):
+    s, h, d = q.shape
+    g = k.shape[1]
+    kd, vd = (t[:pos0 + s].double().repeat_interleave(h // g, 1).transpose(0, 1) for t in (k, v))
+    sc = (q.double().transpose(0, 1) @ kd.transpose(1, 2)) * scale
+    seen = torch.arange(pos0 + s, device=DEV)[None, :] <= pos0 + torch.arange(s, device=DEV)[:, None]
+    return (torch.softmax(sc.masked_fill(~seen, float("-inf")), -1) @ vd).transpose(0, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("s, pos0, h, g, bshd", [(1, 0, 1, 1, True), (16, 0, 4, 2, False), (17, 63, 3, 3, True), (63, 1, 2, 1, True), (64, 64, 2, 2, False),
+                                                 (65, 0, 36, 36, True), (200, 129, 6, 2, True), (777, 0, 4, 4, True)])
+def test_prompt_attention_of_64_wide_heads(s, pos0, h, g, bshd, dtype):
+    """Bound: probabilities carry 2^-16 (bf16) and better, the exponent of a score of magnitude S is off by S 2^-22 at most (fp32 sums of 64
+    products, one multiply, the hardware's exp2): 1e-4 of the largest value here, plus the result's own rounding."""
+    from zhilight_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(s + pos0)
+    n = pos0 + s + 7
+    q = torch.randn(s, h, 64, device=DEV, generator=gen).to(dtype)
+    k, v = (torch.randn(n, g, 64, device=DEV, generator=gen).to(dtype) for _ in range(2))
+    k[pos0 + s:], v[pos0 + s:] = float("nan"), float("inf")     # slots that no query sees hold anything
+    ref = _attention64(q, k, v, pos0, 0.125)
+    lay = (lambda t: t) if bshd else (lambda t: t.transpose(0, 1).contiguous())
+    out = ops.prefill_attention_w32(q, lay(k), lay(v), pos0, g, 0.125, bshd=bshd)
+    assert bool(((out.double() - ref).abs() <= HALF_ULP[dtype] * ref.abs() + 1e-4 * float(ref.abs().max())).all())
+
+
+def test_prompt_attention_of_64_wide_heads_keeps_later_values_out():
+    """a value that is not finite reaches no block of 16 queries before its own"""
+    from zhilight_amd import ops
+    q, k, v = (torch.randn(128, 2, 64, device=DEV).to(torch.bfloat16) for _ in range(3))
+    v[100] = float("inf")
+    out = ops.prefill_attention_w32(q, k, v, 0, 2, 0.125)
+    assert bool(torch.isfinite(out[:96]).all()) and not bool(torch.isfinite(out[100:]).any())
+    for bad in (dict(d=128), dict(d=32)):
+        from zhilight_amd._lib import ZLError
+        with pytest.raises(ZLError):
+            ops.prefill_attention_w32(*(torch.zeros(8, 2, bad["d"], device=DEV, dtype=torch.bfloat16) for _ in range(3)), 0, 2, 0.1)

@@ -27,9 +27,10 @@
 
 namespace {
 
-constexpr int kBQ = 64, kBK = 64, kD = 128;
-constexpr int kKRow = kD + 8;       // K tile row (halfs), padded: conflict-free b128 reads
-constexpr int kVRow = kD + 16;      // V tile row (halfs): 288 B, conflict-free transpose reads
+constexpr int kBQ = 64, kBK = 64;
+// padded tile rows (halfs): K rows of 272 / 144 B for conflict-free b128 reads, V rows of 288 / 160 B for conflict-free transpose reads
+constexpr int k_row(int d) { return d + 8; }
+constexpr int v_row(int d) { return d + 16; }
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
@@ -55,10 +56,13 @@ __device__ __forceinline__ f4 pf_mfma(uint4 a, uint4 b, f4 c) {
 }
 
 // DT = ZL_F16 / ZL_BF16: probabilities are rounded to T for the P.V product (flash-attention arithmetic)
-constexpr int kGroupLds = (kBK * kKRow + kBK * kVRow) * 2;     // one group's K + V tile: 35 840 bytes (>= its 32.5 KB merge record)
+constexpr int group_lds(int d) { return kBK * (k_row(d) + v_row(d)) * 2; }     // one group's K + V tile: 35 840 bytes at D = 128 (>= its 32.5 KB merge record)
 
-template <int DT, int G>
-__global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const PrefillParams p) {
+// W32: the probabilities keep 32-bit quality on their way into P.V: each is split into two numbers of T (the rounded one and the rounded
+// rest: 16 bits of mantissa in bf16, 22 in fp16), multiplied one after the other, and the normaliser sums the unrounded ones
+template <int DT, int G, int D, bool W32>
+__global__ __launch_bounds__(256 * G, G == 1 ? (D == 64 ? 4 : 2) : 4) void k_prefill_attn(const PrefillParams p) {
+    constexpr int kD = D, kKRow = k_row(D), kVRow = v_row(D), kGroupLds = group_lds(D), NT = D / 32, NDB = D / 16;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_pf[];
     const int group = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));     // 4 waves each
     uint16_t* ks = reinterpret_cast<uint16_t*>(smem_pf + (size_t)group * kGroupLds);
@@ -88,17 +92,17 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
     const size_t kv_off = p.bshd ? (size_t)hk * kD : (size_t)hk * p.len_buf * kD;
 
     // Q fragments (B operand of S^T = K.Q^T): column q = lane & 15, k-chunk = d 32 t + 8 kq .. +7
-    uint4 qf[4];
+    uint4 qf[NT];
     {
         const int qr = qrow < p.s_q ? qrow : p.s_q - 1;
         const uint16_t* qp = p.q + ((size_t)qr * p.h + head) * kD + 8 * kq;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) qf[t] = *reinterpret_cast<const uint4*>(qp + 32 * t);
+        for (int t = 0; t < NT; ++t) qf[t] = *reinterpret_cast<const uint4*>(qp + 32 * t);
     }
 
-    f4 o[8];                                              // O block: column d = 16 db + (lane & 15), rows q = 4 kq + i
+    f4 o[NDB];                                            // O block: column d = 16 db + (lane & 15), rows q = 4 kq + i
 #pragma unroll
-    for (int db = 0; db < 8; ++db) o[db] = (f4){0.f, 0.f, 0.f, 0.f};
+    for (int db = 0; db < NDB; ++db) o[db] = (f4){0.f, 0.f, 0.f, 0.f};
     float m_run = -1e20f, l_run = 0.f;                    // per query (lane & 15), replicated over kq
 
     const int last_q = min(q0 + kBQ, p.s_q) - 1;
@@ -120,7 +124,8 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
         const uint16_t* kp_ = p.k + kv_off + (size_t)kc_ * kv_stride;                                     \
         const uint16_t* vp_ = p.v + kv_off + (size_t)kc_ * kv_stride;                                     \
         const bool dead_ = kg_ >= n_keys;                                                                  \
-        ZL_PF_LOAD1(0, kp_, vp_, dead_) ZL_PF_LOAD1(1, kp_, vp_, dead_) ZL_PF_LOAD1(2, kp_, vp_, dead_) ZL_PF_LOAD1(3, kp_, vp_, dead_) \
+        ZL_PF_LOAD1(0, kp_, vp_, dead_) ZL_PF_LOAD1(1, kp_, vp_, dead_)                                    \
+        if constexpr (D == 128) { ZL_PF_LOAD1(2, kp_, vp_, dead_) ZL_PF_LOAD1(3, kp_, vp_, dead_) }        \
     }
     ZL_PF_LOAD(group)
 
@@ -133,7 +138,10 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
 #define ZL_PF_ST(c_)                                                                                       \
         *reinterpret_cast<uint4*>(&ks[skey * kKRow + (sdch + 4 * c_) * 8]) = kr##c_;                       \
         *reinterpret_cast<uint4*>(&vt[skey * kVRow + (sdch + 4 * c_) * 8]) = vr##c_;
-        if (live) { ZL_PF_ST(0) ZL_PF_ST(1) ZL_PF_ST(2) ZL_PF_ST(3) }
+        if (live) {
+            ZL_PF_ST(0) ZL_PF_ST(1)
+            if constexpr (D == 128) { ZL_PF_ST(2) ZL_PF_ST(3) }
+        }
 #undef ZL_PF_ST
         __syncthreads();
         if (!live) continue;
@@ -145,7 +153,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
         for (int kb = 0; kb < 4; ++kb) {
             st[kb] = (f4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
+            for (int t = 0; t < NT; ++t) {
                 const uint4 a = *reinterpret_cast<const uint4*>(&ks[(kb * 16 + nq) * kKRow + 32 * t + 8 * kq]);
                 st[kb] = pf_mfma<DT>(a, qf[t], st[kb]);
             }
@@ -183,7 +191,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         m_run = m_new;
         float lsum = 0.f;
-        uint4 pf[2];                                      // P as the A operand of P.V: k-chunk kq of key group j
+        uint4 pf[2], pl[2];                               // P (W32: and the rest) as the A operand of P.V: k-chunk kq of key group j
         auto cvt = [](float x) -> uint16_t {
             if constexpr (DT == ZL_F16) return __builtin_bit_cast(uint16_t, (_Float16)x);
             else {
@@ -193,18 +201,25 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
         };
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            uint32_t w[4];
+            uint32_t w[4], wl[4];
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
 #pragma unroll
                 for (int i2 = 0; i2 < 2; ++i2) {
-                    const uint16_t p0 = cvt(__builtin_amdgcn_exp2f(st[2 * j + half][2 * i2] - m_new));
-                    const uint16_t p1 = cvt(__builtin_amdgcn_exp2f(st[2 * j + half][2 * i2 + 1] - m_new));
-                    lsum += ZT<DT>::to_f32(p0) + ZT<DT>::to_f32(p1);   // the normaliser sums what the product uses
+                    const float e0 = __builtin_amdgcn_exp2f(st[2 * j + half][2 * i2] - m_new);
+                    const float e1 = __builtin_amdgcn_exp2f(st[2 * j + half][2 * i2 + 1] - m_new);
+                    const uint16_t p0 = cvt(e0), p1 = cvt(e1);
                     w[half * 2 + i2] = (uint32_t)p0 | ((uint32_t)p1 << 16);
+                    if constexpr (W32) {
+                        lsum += e0 + e1;
+                        wl[half * 2 + i2] = (uint32_t)cvt(e0 - ZT<DT>::to_f32(p0)) | ((uint32_t)cvt(e1 - ZT<DT>::to_f32(p1)) << 16);
+                    } else {
+                        lsum += ZT<DT>::to_f32(p0) + ZT<DT>::to_f32(p1);   // the normaliser sums what the product uses
+                    }
                 }
             }
             pf[j] = make_uint4(w[0], w[1], w[2], w[3]);
+            if constexpr (W32) pl[j] = make_uint4(wl[0], wl[1], wl[2], wl[3]);
         }
         l_run = l_run * alpha + lsum;                     // per-lane partial; lanes of a query are merged at the end
         // ---- rescale O: the factor of row q = 4 kq + i comes from the lane whose nq is that row -- only when some row's maximum
@@ -214,7 +229,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
             __builtin_amdgcn_s_waitcnt(0xc07f);           // lgkmcnt(0): the strip write has landed (wave-private)
             const f4 al = *reinterpret_cast<const f4*>(&strip[wave_all][4 * kq]);
 #pragma unroll
-            for (int db = 0; db < 8; ++db) {
+            for (int db = 0; db < NDB; ++db) {
                 o[db][0] *= al[0]; o[db][1] *= al[1]; o[db][2] *= al[2]; o[db][3] *= al[3];
             }
         }
@@ -226,10 +241,22 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
 #pragma unroll
-            for (int db = 0; db < 8; ++db) {
+            for (int db = 0; db < NDB; ++db) {
                 const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)(vtr + (32 * j) * kVRow + 16 * db));
                 const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)(vtr + (32 * j + 16) * kVRow + 16 * db));
-                const s8 b = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                s8 b = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                if constexpr (W32) {
+                    // a value row behind the wave's last query must not reach its rows: its probability is 0, but 0 x inf is not
+                    if (diag) {
+                        const int last = p.pos0 + q0 + wave * 16 + 15 - key0 - 32 * j - 4 * kq;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            if (i > last) b[i] = 0;
+                            if (16 + i > last) b[4 + i] = 0;
+                        }
+                    }
+                    o[db] = pf_mfma<DT>(pl[j], __builtin_bit_cast(uint4, b), o[db]);
+                }
                 o[db] = pf_mfma<DT>(pf[j], __builtin_bit_cast(uint4, b), o[db]);
             }
         }
@@ -244,7 +271,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
         float* rec = reinterpret_cast<float*>(smem_pf + (size_t)group * kGroupLds);     // [wave][16 rows][128] O, then [wave][64 lanes] m, l
         if (group > 0) {
 #pragma unroll
-            for (int db = 0; db < 8; ++db)
+            for (int db = 0; db < NDB; ++db)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) rec[(wave * 16 + 4 * kq + i) * kD + 16 * db + nq] = o[db][i];
             rec[4 * 16 * kD + wave * 64 + lane] = m_run;
@@ -268,7 +295,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
             const f4 f0 = *reinterpret_cast<const f4*>(&strip[wave_all][4 * kq]);
             const f4 fg = *reinterpret_cast<const f4*>(&strip[4 + wave_all][4 * kq]);
 #pragma unroll
-            for (int db = 0; db < 8; ++db)
+            for (int db = 0; db < NDB; ++db)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     o[db][i] = o[db][i] * f0[i] + rg[(wave * 16 + 4 * kq + i) * kD + 16 * db + nq] * fg[i];
@@ -287,7 +314,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 4) void k_prefill_attn(const 
         if (row >= p.s_q) continue;
         uint16_t* op = p.out + ((size_t)row * p.h + head) * kD + nq;
 #pragma unroll
-        for (int db = 0; db < 8; ++db) op[db * 16] = ZT<DT>::from_f32(o[db][i] * inv[i]);
+        for (int db = 0; db < NDB; ++db) op[db * 16] = ZT<DT>::from_f32(o[db][i] * inv[i]);
     }
 }
 
@@ -303,14 +330,14 @@ extern "C" int zl_prefill_attn(const uint16_t* q, const uint16_t* k_buf, const u
     return zl_prefill_attn_ex(q, k_buf, v_buf, out, s_q, pos0, h, hkv, d, scale, len_buf, bshd, dtype, 0, s);
 }
 
-template <int DT, int G>
+template <int DT, int G, int D = 128, bool W32 = false>
 static int launch_prefill(const PrefillParams& p, dim3 grid, hipStream_t hs) {
-    const size_t lds = (size_t)G * kGroupLds + (size_t)4 * G * 16 * sizeof(float);       // tiles + one 64-byte strip per wave
+    const size_t lds = (size_t)G * group_lds(D) + (size_t)4 * G * 16 * sizeof(float);       // tiles + one 64-byte strip per wave
     if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_prefill_attn<DT, G>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_prefill_attn<DT, G, D, W32>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return ZL_ELIMIT;
     }
-    hipLaunchKernelGGL((k_prefill_attn<DT, G>), grid, dim3(256 * G), lds, hs, p);
+    hipLaunchKernelGGL((k_prefill_attn<DT, G, D, W32>), grid, dim3(256 * G), lds, hs, p);
     return zl_launch_status();
 }
 
@@ -321,7 +348,7 @@ extern "C" int zl_prefill_attn_ex(const uint16_t* q, const uint16_t* k_buf, cons
                                   int dtype, int groups, zl_stream_t s) {
     ZL_CHECK_ARG(q && k_buf && v_buf && out && s_q > 0 && pos0 >= 0 && h > 0 && hkv > 0 && len_buf > 0, ZL_EINVAL);
     ZL_CHECK_ARG(h % hkv == 0 && pos0 + s_q <= len_buf, ZL_ESHAPE);
-    ZL_CHECK_ARG(d == kD, ZL_ESHAPE);          // other head sizes: the mask form of zl_decode_attn
+    ZL_CHECK_ARG(d == 128, ZL_ESHAPE);         // 64: zl_prefill_attn_w32; other head sizes: the mask form of zl_decode_attn
     ZL_CHECK_ARG(dtype == ZL_F16 || dtype == ZL_BF16, ZL_EDTYPE);
     ZL_CHECK_ARG(h <= 65535, ZL_ELIMIT);
     const bool plain_map = groups == -1;               // A/B switch: one group, work items in plain dispatch order (the round-4 launch)
@@ -350,4 +377,24 @@ extern "C" int zl_prefill_attn_ex(const uint16_t* q, const uint16_t* k_buf, cons
         default: ZL_PF_G(4)
     }
 #undef ZL_PF_G
+}
+
+// the same for heads of 64 numbers (MiniCPM), where the mask form of zl_decode_attn -- probabilities in fp32, every query row a pass over
+// its keys on the VALU -- was the only kernel: 777 tokens x 36 heads took 1 872 us per layer.  The probabilities keep 32-bit quality here (W32:
+// the second product costs 8 MFMAs per 64 keys and wave, against the key products' 8 and the tile's latency of ~2 us).
+extern "C" int zl_prefill_attn_w32(const uint16_t* q, const uint16_t* k_buf, const uint16_t* v_buf, uint16_t* out, int64_t s_q, int64_t pos0,
+                                   int64_t h, int64_t hkv, int64_t d, float scale, int64_t len_buf, int bshd, int dtype, zl_stream_t s) {
+    ZL_CHECK_ARG(q && k_buf && v_buf && out && s_q > 0 && pos0 >= 0 && h > 0 && hkv > 0 && len_buf > 0, ZL_EINVAL);
+    ZL_CHECK_ARG(h % hkv == 0 && pos0 + s_q <= len_buf && d == 64, ZL_ESHAPE);
+    ZL_CHECK_ARG(((uintptr_t)q & 15) == 0 && ((uintptr_t)k_buf & 15) == 0 && ((uintptr_t)v_buf & 15) == 0, ZL_ESHAPE);
+    ZL_CHECK_ARG(dtype == ZL_F16 || dtype == ZL_BF16, ZL_EDTYPE);
+    ZL_CHECK_ARG(h <= 65535 && s_q < (1 << 30) && len_buf < (1 << 30), ZL_ELIMIT);
+    PrefillParams p;
+    p.q = q; p.k = k_buf; p.v = v_buf; p.out = out;
+    p.s_q = (int)s_q; p.pos0 = (int)pos0; p.h = (int)h; p.hkv = (int)hkv; p.n_rep = (int)(h / hkv);
+    p.len_buf = (int)len_buf; p.bshd = bshd; p.scale = scale; p.pair = 0;
+    p.nx = (int)((s_q + kBQ - 1) / kBQ);
+    ZL_CHECK_ARG((int64_t)p.nx * h < ((int64_t)1 << 31), ZL_ELIMIT);
+    const dim3 grid((unsigned)(p.nx * (int)h));
+    return dtype == ZL_F16 ? launch_prefill<ZL_F16, 1, 64, true>(p, grid, (hipStream_t)s) : launch_prefill<ZL_BF16, 1, 64, true>(p, grid, (hipStream_t)s);
 }

@@ -1269,6 +1269,10 @@ class LLaMA:
             return ops.rope_cos_sin_yarn(pos, c.dim_head, c.rope_theta, rs["factor"], low, high, msc)
         raise ops.ZLError(f"rope_scaling type {kind!r} is not supported (supported: llama3, dynamic, yarn)")
 
+    def _prompt_attention(self):
+        """the matrix-core prompt attention of this head size, None where there is none (then the mask form runs)"""
+        return {128: ops.prefill_attention, 64: ops.prefill_attention_w32}.get(self.cfg.dim_head)
+
     def _prefill_mask(self, s, len_buf, pos0=0):
         """causal mask + workspace for head sizes the MFMA prefill kernel does not cover"""
         key = ("prefill", s, len_buf, pos0)
@@ -1332,6 +1336,7 @@ class LLaMA:
         cos, sin = self._rope_tables(pos)
         buf_lens = ctx.buf_lens[task:task + 1]
         scale = 1.0 / math.sqrt(c.dim_head)
+        prompt_attn = self._prompt_attention()
         main = torch.cuda.current_stream(dev)
         if "reduce_stream" not in self._bufs:
             self._bufs["reduce_stream"] = torch.cuda.Stream(device=dev, priority=int(os.environ.get("DUAL_STREAM_PRIORITY", "-1")))
@@ -1367,9 +1372,9 @@ class LLaMA:
                 q, kr, v = ops.rope_qk_cache(cos[a:b], sin[a:b], qkv, c.num_heads, c.num_kv_heads, c.dim_head, True)
                 ops.copy_to_rag_buffer2(pos[a:b].view(1, n), buf_lens, kr.view(1, n, c.num_kv_heads, c.dim_head),
                                         v.view(1, n, c.num_kv_heads, c.dim_head), ka, va)
-                if c.dim_head == 128:
-                    att = ops.prefill_attention(q.view(n, c.num_heads, c.dim_head), ctx.kv[task][li, 0], ctx.kv[task][li, 1],
-                                                pos0 + a, c.num_kv_heads, scale)
+                if prompt_attn:
+                    att = prompt_attn(q.view(n, c.num_heads, c.dim_head), ctx.kv[task][li, 0], ctx.kv[task][li, 1],
+                                      pos0 + a, c.num_kv_heads, scale)
                 else:
                     mask, ws = self._prefill_mask(n, ctx.max_len_buf, pos0 + a)
                     att = ops.multi_query_attention_rag_buffer(q.view(1, n, c.num_heads, c.dim_head), buf_lens, ka, va, mask,
@@ -1396,8 +1401,8 @@ class LLaMA:
         (tokens <- greedy first token, positions = placement = S, valid_lens = S + 1) and returns the logits of
         the last prompt position (1, vocab).  Sequence: separate RMSNorm, W4A16 GEMM (M = S: the M-tiled MFMA
         kernel, the arithmetic of the reference's M > 40 dequant + GEMM branch), rope_qk_cache,
-        copy_to_rag_buffer2, causal MFMA attention (prefill_attention; other head sizes: the mask form of
-        multi_query_attention_rag_buffer)."""
+        copy_to_rag_buffer2, causal MFMA attention (prefill_attention, 64-wide heads prefill_attention_w32; other head sizes: the
+        mask form of multi_query_attention_rag_buffer)."""
         c, dev = self.cfg, self.device
         s = int(prompt.numel())
         if s < 1 or pos0 + s + 1 > ctx.max_len_buf:
@@ -1414,6 +1419,7 @@ class LLaMA:
         placement = pos.view(1, s)
         buf_lens = ctx.buf_lens[task:task + 1]
         scale = 1.0 / math.sqrt(c.dim_head)
+        prompt_attn = self._prompt_attention()
         for li, layer in enumerate(self.layers):
             ka, va = ctx.k_addrs[li][task:task + 1], ctx.v_addrs[li][task:task + 1]
             qkv = layer.project_qkv(hidden, c.eps)
@@ -1431,15 +1437,15 @@ class LLaMA:
                     tl = torch.tensor([tk.shape[0]], dtype=torch.int32, device=dev)
                     ops.copy_to_rag_buffer2(placement, tl, k3.view(1, s, c.num_kv_heads, c.dim_head), v3.view(1, s, c.num_kv_heads, c.dim_head),
                                             ops.make_ptr_table([tk]), ops.make_ptr_table([tv]))
-                    if c.dim_head == 128:
-                        att = ops.prefill_attention(q.view(s, c.num_heads, c.dim_head), tk, tv, pos0, c.num_kv_heads, scale)
+                    if prompt_attn:
+                        att = prompt_attn(q.view(s, c.num_heads, c.dim_head), tk, tv, pos0, c.num_kv_heads, scale)
                     else:
                         mask, ws = self._prefill_mask(s, tk.shape[0], pos0)
                         att = ops.multi_query_attention_rag_buffer(q.view(1, s, c.num_heads, c.dim_head), tl, ops.make_ptr_table([tk]),
                                                                    ops.make_ptr_table([tv]), mask, scale, tk.shape[0], c.num_kv_heads,
                                                                    workspace=ws)
-                elif c.dim_head == 128:
-                    att = ops.prefill_attention(q.view(s, c.num_heads, c.dim_head), k3, v3, 0, c.num_kv_heads, scale)
+                elif prompt_attn:
+                    att = prompt_attn(q.view(s, c.num_heads, c.dim_head), k3, v3, 0, c.num_kv_heads, scale)
                 else:
                     mask, ws = self._prefill_mask(s, s, 0)
                     att = ops.multi_query_attention_rag_buffer(
@@ -1450,9 +1456,8 @@ class LLaMA:
                 continue
             ops.copy_to_rag_buffer2(placement, buf_lens, k.view(1, s, c.num_kv_heads, c.dim_head),
                                     v.view(1, s, c.num_kv_heads, c.dim_head), ka, va)
-            if c.dim_head == 128:
-                att = ops.prefill_attention(q.view(s, c.num_heads, c.dim_head), ctx.kv[task][li, 0], ctx.kv[task][li, 1], pos0,
-                                            c.num_kv_heads, scale)
+            if prompt_attn:
+                att = prompt_attn(q.view(s, c.num_heads, c.dim_head), ctx.kv[task][li, 0], ctx.kv[task][li, 1], pos0, c.num_kv_heads, scale)
             else:
                 mask, ws = self._prefill_mask(s, ctx.max_len_buf, pos0)
                 att = ops.multi_query_attention_rag_buffer(q.view(1, s, c.num_heads, c.dim_head), buf_lens, ka, va, mask,

@@ -1239,6 +1239,20 @@ def prefill_attention(q, k_buf, v_buf, pos0, num_kv_heads, scale, bshd=True, out
     return out
 
 
+def prefill_attention_w32(q, k_buf, v_buf, pos0, num_kv_heads, scale, bshd=True, out=None):
+    """prefill_attention for heads of 64 numbers, probabilities in 32-bit quality (what the mask form of multi_query_attention_rag_buffer gives)."""
+    _chk_cuda(q, k_buf, v_buf)
+    if q.dtype not in (torch.float16, torch.bfloat16):
+        raise ZLError("prefill_attention_w32: fp16 / bf16 only")
+    s_q, h, d = q.shape
+    len_buf = k_buf.shape[0] if bshd else k_buf.shape[1]
+    if out is None:
+        out = torch.empty_like(q)
+    check(lib().zl_prefill_attn_w32(_p(q), _p(k_buf), _p(v_buf), _p(out), _i(s_q), _i(pos0), _i(h), _i(num_kv_heads), _i(d), _f(scale), _i(len_buf),
+                                    C.c_int(int(bshd)), C.c_int(_dt(q)), _stream()), "prefill_attn_w32")
+    return out
+
+
 def element_add_scale(a, b, scale=1.0, scale_residual=True, out=None):
     """nn::element_add_scale_out (src/nn/block/block_kernel.cu:19-50)."""
     _chk_cuda(a, b)
