@@ -705,6 +705,14 @@ int zl_rmsnorm_quant(const uint16_t* x, const uint16_t* weight, uint16_t* out, i
                      int64_t rows, int64_t dim, float eps, float scale, int dtype, zl_stream_t s);
 int zl_int8_gemm_nt(const int8_t* a /* (M,K) */, const int8_t* b /* (N,K) */, int32_t* c /* (M,N) */,
                     int64_t m, int64_t n, int64_t k, zl_stream_t s);
+/* the INT8 linear of a prompt chunk (m > 32, k % 128 == 0, a / b / b2 16-byte and out 8-byte aligned; otherwise ZL_ESHAPE) in one launch:
+ * zl_int8_gemm_nt and, while the sums are in registers, with the same bits as the separate calls,
+ *   b2 == NULL, addend == NULL   zl_quant_scale_back
+ *   b2 == NULL, addend           zl_quant_back_element_add_scale (out may alias addend)
+ *   b2, sy2                      zl_quant_back_act_mul of the products with b (gate) and b2 (up), n rows each; act 0 silu, 1 gelu
+ * act is -1 without b2. */
+int zl_int8_linear(const int8_t* a, const float* sx, const int8_t* b, const uint16_t* sy, const int8_t* b2, const uint16_t* sy2,
+                   const uint16_t* addend, uint16_t* out, int64_t m, int64_t n, int64_t k, float scale, int act, int dtype, zl_stream_t s);
 int zl_quant_scale_back(const int32_t* c, const float* scale_x, const uint16_t* scale_y, uint16_t* out,
                         int64_t m, int64_t n, int dtype, zl_stream_t s);
 int zl_quant_back_act_mul(const int32_t* a, const float* a_sx, const uint16_t* a_sy, const int32_t* b,

@@ -110,3 +110,21 @@ def test_prompt_attention_of_64_wide_heads_keeps_later_values_out():
         from zhilight_amd._lib import ZLError
         with pytest.raises(ZLError):
             ops.prefill_attention_w32(*(torch.zeros(8, 2, bad["d"], device=DEV, dtype=torch.bfloat16) for _ in range(3)), 0, 2, 0.1)
+
+
+# ---- INT8 linears of prompt chunks (zl_int8_linear): the bits of the separate calls -----------------------------------------------------
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m, n, k", [(33, 16, 128), (64, 100, 256), (100, 1001, 384), (257, 514, 128), (1000, 2048, 256), (1025, 6144, 128), (2049, 4100, 128)])
+def test_int8_linear(m, n, k, dtype):
+    from zhilight_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(m)
+    a, b, b2 = (torch.randint(-127, 128, (r, k), device=DEV, generator=g, dtype=torch.int8) for r in (m, n, n))
+    sx = torch.rand(m, device=DEV, generator=g) * 0.02
+    sy, sy2 = (torch.rand(n, device=DEV, generator=g).mul(0.02).to(dtype) for _ in range(2))
+    c, c2 = ((a.double() @ w.double().T).round().to(torch.int32) for w in (b, b2))
+    assert torch.equal(ops.int8_gemm_nt(a, b), c)
+    assert torch.equal(ops.int8_linear(a, sx, b, sy, dtype=dtype), ops.quant_scale_back(c, sx, sy, dtype))
+    assert torch.equal(ops.int8_linear(a, sx, b, sy, b2, sy2, dtype=dtype), ops.quant_back_act_mul(c, sx, sy, c2, sx, sy2, "silu", dtype))
+    add = torch.randn(m, n, device=DEV, generator=g).to(dtype)
+    want = ops.quant_back_element_add_scale(c, sx, sy, add, 0.5)
+    assert torch.equal(ops.int8_linear(a, sx, b, sy, addend=add, scale=0.5, out=add), want)

@@ -245,7 +245,7 @@ extern "C" int zl_gemm_nt(const uint16_t* x, int64_t ldx, const uint16_t* w, con
     const unsigned gx = (unsigned)((n + kDBN - 1) / kDBN);
     hipStream_t hs = (hipStream_t)s;
     if (m > 32 && m < (1 << 30) && n < (1 << 30) && g16_takes(x, ldx, w, k, k)) {
-        const Gemm16P g = {x, w, ldx, k, (int)m, (int)n, (int)k, 0, 0, (int)k};
+        const Gemm16P g = {x, w, ldx, k, (int)m, (int)n, (int)k, 0, 0, (int)k, nullptr, 0};
         const int vec = n % 4 == 0 && ((uintptr_t)y & 7) == 0;
         if (dtype == ZL_F16) return g16_launch<ZL_F16>(g, DenseEpi<ZL_F16>{y, bias, alpha, vec}, hs);
         return g16_launch<ZL_BF16>(g, DenseEpi<ZL_BF16>{y, bias, alpha, vec}, hs);

@@ -6,6 +6,7 @@
 //   quant_scale_back            src/nn/quant/int8/quant_kernel.cu:231-246
 //   quant_back_act_mul          src/nn/quant/int8/quant_kernel.cu:589-614
 #include "zl_common.h"
+#include "zl_gemm16.h"
 
 namespace {
 
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(256) void k_int8_gemm(const int8_t* __restrict__ a,
         }
 }
 
-// Tiled int8 GEMM (the Int8Linear hot kernel, functions::Gemm int8 path of linear.cpp:557-635 / cuBLASLt IMMA):
+// Tiled int8 GEMM for up to 32 rows (more: zl_gemm16.h; the Int8Linear hot kernel, functions::Gemm int8 path of linear.cpp:557-635 / cuBLASLt IMMA):
 // same structure as dense_gemm.hip -- workgroup = 4 waves = BM x 128 outputs, wave = BM x 32, K in 256-byte
 // chunks, the activation chunk double-buffered in LDS, weight fragments (lane = row n, 16 consecutive k) loaded
 // two chunks ahead straight into the MFMA B registers (v_mfma_i32_16x16x64_i8).  Few workgroups (decode
@@ -411,6 +412,89 @@ __global__ void k_scale_back_ex(const BackParams p) {
     }
 }
 
+// ---- the large tiles of zl_gemm16.h (more than 32 rows: prompt chunks)
+struct I8RawEpi {                                              // the int32 sums
+    int32_t* c;
+    int vec;                                                   // rows in 16-byte pieces
+    template <int NI, class F>
+    __device__ __forceinline__ void row(int r, int c0, int n, F sum) const {
+        int32_t* cr = c + (size_t)r * n;
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            const int col = c0 + 16 * j;
+            const v4i v = sum(j);
+            if (vec && col + 4 <= n) *reinterpret_cast<v4i*>(cr + col) = v;
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (col + e < n) cr[col + e] = v[e];
+        }
+    }
+};
+
+// quant_scale_back / quant_back_element_add_scale / quant_back_act_mul on the sums while they are in registers: what k_scale_back,
+// k_scale_back_ex<kBackAdd> and k_back_act_mul compute, expression by expression (the same bits)
+template <int DT, bool GATED>
+struct I8BackEpi {
+    const float* sx; const uint16_t* sy; const uint16_t* sy2; const uint16_t* addend; uint16_t* out;
+    float scale;
+    int cols, act;                                             // output columns; GATED: 0 silu, 1 gelu
+    __device__ __forceinline__ void put4(int r, int col, const float (&v)[4]) const {
+        uint16_t* o = out + (size_t)r * cols + col;
+        if (cols % 4 == 0 && col + 4 <= cols) {
+            uint32_t h[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = ZT<DT>::from_f32(v[e]);
+            *reinterpret_cast<uint2*>(o) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (col + e < cols) o[e] = ZT<DT>::from_f32(v[e]);
+        }
+    }
+    template <int NI, class F>
+    __device__ __forceinline__ void row(int r, int c0, int n, F sum) const {
+        const float x = sx[r];
+        if constexpr (GATED) {
+#pragma unroll
+            for (int j = 0; j < NI; j += 2) {
+                const int c = c0 + 16 * j, col = (c >> 5) * 16 + (c & 15);                // (c: in the paired blocks' numbering)
+                const v4i a = sum(j), b = sum(j + 1);
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int k = min(col + e, cols - 1);
+                    const float ab = (float)a[e] * x * ZT<DT>::to_f32(sy[k]), bb = (float)b[e] * x * ZT<DT>::to_f32(sy2[k]);
+                    float gate;
+                    if (act == 0) gate = ab / (1.0f + expf(-ab));
+                    else gate = 0.5f * ab * (1.0f + tanhf(0.7978845608028654f * ab * (1.0f + 0.044715f * ab * ab)));
+                    v[e] = bb * gate;
+                }
+                if (col < cols) put4(r, col, v);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NI; ++j) {
+                const int col = c0 + 16 * j;
+                if (col >= cols) continue;
+                const v4i a = sum(j);
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int k = min(col + e, cols - 1);
+                    v[e] = (float)a[e] * x * ZT<DT>::to_f32(sy[k]);
+                    if (addend) v[e] = (v[e] + ZT<DT>::to_f32(addend[(size_t)r * cols + k])) * scale;
+                }
+                put4(r, col, v);
+            }
+        }
+    }
+};
+
+static inline bool i8_takes(const int8_t* a, const int8_t* b, const int8_t* b2, int64_t m, int64_t n, int64_t k) {
+    return m > 32 && m < (1 << 30) && n < (1 << 29) && k % 128 == 0 && k <= (1 << 22) && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)b2) & 15) == 0;
+}
+
 template <int MODE>
 int launch_back(const BackParams& p, int dtype, hipStream_t st) {
     if (p.rows > 65535) return ZL_ELIMIT;
@@ -466,8 +550,10 @@ int zl_int8_gemm_nt(const int8_t* a, const int8_t* b, int32_t* c, int64_t m, int
     ZL_CHECK_ARG(a && b && c && m > 0 && n > 0 && k > 0, ZL_EINVAL);
     ZL_CHECK_ARG(k % 16 == 0, ZL_ESHAPE);
     hipStream_t hs0 = (hipStream_t)s;
+    if (i8_takes(a, b, nullptr, m, n, k))
+        return g16_launch<G16_I8>(Gemm16P{a, b, k, k, (int)m, (int)n, (int)k, 0, 0, (int)k, nullptr, 0}, I8RawEpi{c, n % 4 == 0 && ((uintptr_t)c & 15) == 0}, hs0);
     if (k % 256 == 0 && ((uintptr_t)a & 15) == 0 && ((uintptr_t)b & 15) == 0) {
-        const int bm = m <= 16 ? 16 : (m <= 32 ? 32 : 64);
+        const int bm = m <= 16 ? 16 : 32;
         const int gxt = (int)((n + 127) / 128), gyt = (int)((m + bm - 1) / bm);
         ZL_CHECK_ARG(gyt <= 65535, ZL_ELIMIT);
         const int chunks = (int)(k / 256);
@@ -488,8 +574,7 @@ int zl_int8_gemm_nt(const int8_t* a, const int8_t* b, int32_t* c, int64_t m, int
         }
         const dim3 grid((unsigned)gxt, (unsigned)gyt, (unsigned)splits);
         if (bm == 16) hipLaunchKernelGGL(k_int8_gemm_tiled<16>, grid, dim3(256), 0, hs0, a, b, c, (int)m, (int)n, (int)k, chunks, sc, splits > 1);
-        else if (bm == 32) hipLaunchKernelGGL(k_int8_gemm_tiled<32>, grid, dim3(256), 0, hs0, a, b, c, (int)m, (int)n, (int)k, chunks, sc, splits > 1);
-        else hipLaunchKernelGGL(k_int8_gemm_tiled<64>, grid, dim3(256), 0, hs0, a, b, c, (int)m, (int)n, (int)k, chunks, sc, splits > 1);
+        else hipLaunchKernelGGL(k_int8_gemm_tiled<32>, grid, dim3(256), 0, hs0, a, b, c, (int)m, (int)n, (int)k, chunks, sc, splits > 1);
         return zl_launch_status();
     }
     const int mt = m > 48 ? 4 : (m > 32 ? 3 : (m > 16 ? 2 : 1));
@@ -512,6 +597,23 @@ int zl_int8_gemm_nt(const int8_t* a, const int8_t* b, int32_t* c, int64_t m, int
         default: hipLaunchKernelGGL(k_int8_gemm<4>, grid, dim3(256), 0, hs, a, b, c, (int)m, (int)n, (int)k, kps, splitk > 1); break;
     }
     return zl_launch_status();
+}
+
+// the INT8 linear of a prompt chunk in one launch: the product and its scale-back (see zhilight_amd.h)
+int zl_int8_linear(const int8_t* a, const float* sx, const int8_t* b, const uint16_t* sy, const int8_t* b2, const uint16_t* sy2,
+                   const uint16_t* addend, uint16_t* out, int64_t m, int64_t n, int64_t k, float scale, int act, int dtype, zl_stream_t s) {
+    ZL_CHECK_ARG(a && sx && b && sy && out && m > 0 && n > 0 && k > 0, ZL_EINVAL);
+    ZL_CHECK_ARG((b2 != nullptr) == (sy2 != nullptr) && (b2 ? (act == 0 || act == 1) && !addend : act == -1), ZL_EINVAL);
+    ZL_CHECK_ARG(i8_takes(a, b, b2, m, n, k) && ((uintptr_t)out & 7) == 0, ZL_ESHAPE);
+    ZL_CHECK_ARG(dtype == ZL_F16 || dtype == ZL_BF16, ZL_EDTYPE);
+    const Gemm16P g = {a, b, k, k, (int)m, (int)(b2 ? (n + 15) / 16 * 32 : n), (int)k, 0, 0, (int)k, b2, (int)n};
+    hipStream_t hs = (hipStream_t)s;
+    if (b2) {
+        if (dtype == ZL_F16) return g16_launch<G16_I8, true>(g, I8BackEpi<ZL_F16, true>{sx, sy, sy2, nullptr, out, 1.f, (int)n, act}, hs);
+        return g16_launch<G16_I8, true>(g, I8BackEpi<ZL_BF16, true>{sx, sy, sy2, nullptr, out, 1.f, (int)n, act}, hs);
+    }
+    if (dtype == ZL_F16) return g16_launch<G16_I8>(g, I8BackEpi<ZL_F16, false>{sx, sy, nullptr, addend, out, scale, (int)n, 0}, hs);
+    return g16_launch<G16_I8>(g, I8BackEpi<ZL_BF16, false>{sx, sy, nullptr, addend, out, scale, (int)n, 0}, hs);
 }
 
 int zl_quant_scale_back(const int32_t* c, const float* scale_x, const uint16_t* scale_y, uint16_t* out, int64_t m,

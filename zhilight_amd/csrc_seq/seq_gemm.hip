@@ -434,8 +434,7 @@ template <int DT, int ODT, int EPI = 0>
 void launch_tiled(const GemmP& p, hipStream_t hs) {
     if constexpr (DT == ZL_BF16) {
         if (!p.x_rows && !p.w_rows && !p.tiles && p.k_part % 64 == 0 && g16_takes(p.x, p.ldx, p.w, p.ldw, p.k)) {
-            const Gemm16P g = {reinterpret_cast<const uint16_t*>(p.x), reinterpret_cast<const uint16_t*>(p.w), p.ldx, p.ldw, p.m, p.n, p.k, 0, 0,
-                               p.part ? p.k_part : p.k};
+            const Gemm16P g = {p.x, p.w, p.ldx, p.ldw, p.m, p.n, p.k, 0, 0, p.part ? p.k_part : p.k, nullptr, 0};
             const int vec = p.ldy % 4 == 0 && ((uintptr_t)p.y & 15) == 0;
             const int rc = p.part ? g16_launch<ZL_BF16>(g, PartEpi{p.part, p.m}, hs) : g16_launch<ZL_BF16>(g, SeqEpi<DT, ODT, EPI>{p, vec}, hs);
             if (rc == ZL_OK && p.part)

@@ -531,7 +531,8 @@ class Int8EncoderLayer:
 
     # Decode batches (<= 32 rows): the streaming int8 kernel with the scale-back fused in its epilogue
     # (zl_w8a8_gemm_phase: 4 GEMM launches per layer instead of 5 GEMMs + 4 scale-back kernels + split-K memsets;
-    # bit-identical results).  More rows: the tiled int8 GEMM + the reference's separate scale-back kernels.
+    # bit-identical results).  More rows: the large tiles with the same fusion (zl_int8_linear), the reference's separate scale-back
+    # kernels only where k is no whole 128s.
     @staticmethod
     def _stream(rows):
         return rows <= 32 and os.environ.get("ZL_W8_PHASE", "1") != "0"
@@ -546,13 +547,23 @@ class Int8EncoderLayer:
         _, xq, sx = ops.layernorm_quant(hidden, self.ln_attn, eps)
         if self._stream(hidden.shape[0]):
             return ops.w8a8_gemm_phase(xq, sx, self.qkv.stream_weight(), ops.W8_BACK, out=out, dtype=hidden.dtype)
+        if ops.int8_linear_ok(*xq.shape):
+            return ops.int8_linear(xq, sx, self.qkv.weight, self.qkv.scale, dtype=hidden.dtype, out=out)
         return ops.quant_scale_back(self.qkv.gemm(xq), sx, self.qkv.scale, hidden.dtype, out=out)
 
     def attn_out_add(self, attn, hidden):
         aq, sa = ops.quant_calc_scale(attn)
         if self._stream(hidden.shape[0]):
             return ops.w8a8_gemm_phase(aq, sa, self.attn_out.stream_weight(), ops.W8_BACK_ADD, addend=hidden, scale=1.0, out=hidden)
-        ops.quant_back_element_add_scale(self.attn_out.gemm(aq), sa, self.attn_out.scale, hidden, 1.0, out=hidden)
+        self._add_product(self.attn_out, aq, sa, hidden)
+
+    @staticmethod
+    def _add_product(lin, xq, sx, hidden):
+        """hidden += lin(xq) in place (more than 32 rows)"""
+        if ops.int8_linear_ok(*xq.shape):
+            ops.int8_linear(xq, sx, lin.weight, lin.scale, addend=hidden, out=hidden)
+        else:
+            ops.quant_back_element_add_scale(lin.gemm(xq), sx, lin.scale, hidden, 1.0, out=hidden)
 
     def ff_add(self, hidden, eps, act_buf=None):
         _, xq, sx = ops.layernorm_quant(hidden, self.ln_ff, eps)
@@ -560,10 +571,13 @@ class Int8EncoderLayer:
             act = ops.w8a8_gemm_phase(xq, sx, self._gated_stream_weight(), ops.W8_ACT_SILU, out=act_buf, dtype=hidden.dtype)
             aq, sa = ops.quant_calc_scale(act)
             return ops.w8a8_gemm_phase(aq, sa, self.w_out.stream_weight(), ops.W8_BACK_ADD, addend=hidden, scale=1.0, out=hidden)
-        act = ops.quant_back_act_mul(self.w_in.gemm(xq), sx, self.w_in.scale, self.w_gated.gemm(xq), sx, self.w_gated.scale,
-                                     "silu", hidden.dtype)
+        if ops.int8_linear_ok(*xq.shape):
+            act = ops.int8_linear(xq, sx, self.w_in.weight, self.w_in.scale, self.w_gated.weight, self.w_gated.scale, dtype=hidden.dtype)
+        else:
+            act = ops.quant_back_act_mul(self.w_in.gemm(xq), sx, self.w_in.scale, self.w_gated.gemm(xq), sx, self.w_gated.scale,
+                                         "silu", hidden.dtype)
         aq, sa = ops.quant_calc_scale(act)
-        ops.quant_back_element_add_scale(self.w_out.gemm(aq), sa, self.w_out.scale, hidden, 1.0, out=hidden)
+        self._add_product(self.w_out, aq, sa, hidden)
 
 
 # decode attention with the split merge inside its launch (zl_decode_attn_la): default of the ZL_ATTN_LA switch

@@ -1417,6 +1417,30 @@ def int8_gemm_nt(a, b, out=None):
     return c
 
 
+def int8_linear_ok(m, k):
+    """whether int8_linear takes a product of m rows of k numbers (prompt chunks)"""
+    return m > 32 and k % 128 == 0 and k <= 1 << 22
+
+
+def int8_linear(a, scale_x, b, scale_y, up=None, up_scale=None, addend=None, scale=1.0, act="silu", dtype=torch.float16, out=None):
+    """int8_gemm_nt and its scale-back in one launch, the bits of the separate calls: quant_scale_back, with `addend`
+    quant_back_element_add_scale (out may be the addend), with `up` / `up_scale` quant_back_act_mul of both products.  See int8_linear_ok."""
+    _chk_cuda(a, scale_x, b, scale_y, up, up_scale, addend)
+    m, k = a.shape
+    n = b.shape[0]
+    if b.shape[1] != k or (up is not None and tuple(up.shape) != (n, k)):
+        raise ZLError("size K mismatch")
+    if addend is not None:
+        dtype = addend.dtype
+    if out is None:
+        out = torch.empty((m, n), dtype=dtype, device=a.device)
+    else:
+        _chk_out(out, m, n, dtype, a.device, "int8_linear")
+    check(lib().zl_int8_linear(_p(a), _p(scale_x), _p(b), _p(scale_y), _p(up), _p(up_scale), _p(addend), _p(out), _i(m), _i(n), _i(k), _f(scale),
+                               C.c_int(-1 if up is None else 0 if act == "silu" else 1), C.c_int(_dt(out)), _stream()), "int8_linear")
+    return out
+
+
 def quant_scale_back(c, scale_x, scale_y, dtype=torch.float16, out=None):
     """int8_op::quant_scale_back (src/nn/quant/int8/quant_kernel.cu:248-306)."""
     _chk_cuda(c, scale_x, scale_y)
