@@ -7,6 +7,7 @@
 //                     dt, the decay and the state are fp32.  The same kernel runs linear attention with a scalar decay per head and token
 //                     (zls_decay_scan: x = v, B = k, C = q from columns of one projection, the decay and input scale given per token or
 //                     constant per head, optionally one more value column of ones that carries the normaliser).
+// k_scan_rows         the same scan where the state comes in whole 64s of rows and 16s of columns: token rows by LDS-DMA, four columns per lane
 // k_gated_group_norm  y * silu(z), then each of the row's equal parts divided by its own root mean square, times the weight
 #include "seq_common.h"
 
@@ -211,6 +212,198 @@ __global__ __launch_bounds__(MAXT) void k_ssm_scan(const ScanP p, const zls_batc
     if (p.mode == 1 && tid == 0 && !p.vec) p.seg_prod[seg_at] = prod;
 }
 
+// The scan for states of whole 64s of rows and value widths of whole 16s (what k_ssm_scan above computes; it keeps every other size).
+// A wave owns 16 value columns: lane = (group cg of 4 columns, g of 16), holding states 64 q + 4 g + e, e < 4, of its 4 columns.  What bounds
+// k_ssm_scan is not the recurrence but what surrounds it: 25 16-byte LDS reads per token and wave (a lane reads B, C and the decays of
+// its 32 states for ONE column; here for four: 7), two __shfl_xor through LDS, scalar spills, and a register file that holds 64 offsets
+// and 32 prefetched numbers (2 waves per SIMD).  Here token rows [x | B | C | decays] go global -> LDS by LDS-DMA, a chunk of CH tokens
+// ahead in a second buffer, one barrier per chunk; the sums over g are four DPP rotations; lane g keeps the outputs of the chunk's token g,
+// so stores leave once per chunk.
+// STATE_ONLY: mode 1 (a segment's end state and decay product from a zero state), nothing is read from or multiplied with C.
+// Measured per layer (both passes and the start states between them): (1300, 767, 885) tokens, 16 heads of 128 x 128, decays per channel
+// 937 -> 195 us; 2048 tokens, 64 heads of 64 x 128 623 -> 212 us; single tokens of 8 sequences, 128 such heads 53 -> 18 us (67 MB of state).
+__device__ __forceinline__ void scan_dma(const char* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "m0");
+}
+template <int N>
+__device__ __forceinline__ float row16_ror(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + N, 0xf, 0xf, false));
+}
+
+template <int Q, bool VEC, int CH, bool STATE_ONLY>
+__global__ __launch_bounds__(Q == 4 ? 512 : 1024) void k_scan_rows(const ScanP p, const zls_batch_t b) {
+    constexpr int N = 64 * Q;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int P = p.vdim, WL = P + (2 + VEC) * N, U = WL >> 2;
+    float* dts = lds + 2 * CH * WL;                // [2][CH] (input scale, decay)
+    const int sq = blockIdx.x / p.n_seg, seg = blockIdx.x % p.n_seg, h = blockIdx.y, tid = threadIdx.x, nw = blockDim.x >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane & 15, col = wave * 16 + (lane >> 4) * 4;
+    const bool lin = p.kind == 1;
+    const int grp = lin ? 0 : h / (p.heads / p.groups), inner = p.heads * P;
+    const int64_t chan = lin ? p.ld : inner + 2 * p.groups * N;
+    const int whole = b.seq_start[sq + 1] - b.seq_start[sq];
+    if (seg * p.seg_len >= whole) return;                               // (workgroup-uniform)
+    const int first = b.seq_start[sq] + seg * p.seg_len, count = min(p.seg_len, whole - seg * p.seg_len);
+    const bool last_seg = (seg + 1) * p.seg_len >= whole;
+    if (STATE_ONLY && last_seg) return;                                 // nobody starts from the last segment's end state
+    // a staged row's 16-byte units, 64 per load: where unit lane + 64 r of token `first` lies and how far the next token's is
+    const char* src[4];
+    int64_t step[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int e = min(lane + 64 * r, U - 1) * 4;
+        const float* base = lin ? p.proj : p.xbc;
+        int64_t at, ld = chan;
+        if (e < P) at = lin ? p.v_col0 + h * P + e : h * P + e;
+        else if (e < P + N) at = lin ? p.k_col0 + h * N + e - P : inner + grp * N + e - P;
+        else if (e < P + 2 * N) at = lin ? p.q_col0 + h * N + e - P - N : inner + (p.groups + grp) * N + e - P - N;
+        else { base = p.decay_v; ld = (int64_t)p.heads * N; at = h * N + e - P - 2 * N; }
+        src[r] = reinterpret_cast<const char*>(base + (int64_t)first * ld + at);
+        step[r] = ld * 4;
+    }
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) void*)lds;
+    auto stage = [&](int c0, int buf) {            // a wave's tokens: wave, wave + nw, ...
+        for (int i = wave; i < min(CH, count - c0); i += nw) {
+            const int64_t tok = c0 + i;
+            const uint32_t row = lds0 + (uint32_t)((buf * CH + i) * WL) * 4;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (lane + 64 * r < U) scan_dma(src[r] + tok * step[r], row + r * 1024);
+        }
+    };
+    float* st = p.state + ((size_t)b.seq_slot[sq] * p.heads + h) * N * P;
+    const size_t seg_at = ((size_t)sq * p.n_seg + seg) * p.heads + h;
+    const float rate = lin ? 0.f : expf(p.a_log[h]), bias = lin ? 0.f : p.dt_bias[h], dskip = lin ? 0.f : p.d[h];
+    const float dec_h = (lin && !p.decay_t && p.decay_h) ? p.decay_h[h] : 1.0f;
+    float pre_dt = 0.f, pre_dec = 0.f;
+    auto fetch = [&](int c0) {
+        if (tid < CH) {
+            const size_t tok = (size_t)(first + min(c0 + tid, count - 1));
+            if (lin) {
+                pre_dt = p.gain_t ? p.gain_t[tok * p.heads + h] : 1.0f;
+                pre_dec = p.decay_t ? p.decay_t[tok * p.heads + h] : dec_h;
+            } else {
+                pre_dt = p.proj[tok * p.ld + p.dt_col0 + h];
+            }
+        }
+    };
+    stage(0, 0);
+    fetch(0);
+    float S[4 * Q][4];
+    if (STATE_ONLY) {
+#pragma unroll
+        for (int j = 0; j < 4 * Q; ++j)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) S[j][c] = 0.f;
+    } else {
+        const float* init = (p.mode == 2 && seg > 0) ? p.seg_init + seg_at * N * P : st;
+#pragma unroll
+        for (int j = 0; j < 4 * Q; ++j) {
+            const float4 v = *reinterpret_cast<const float4*>(init + (size_t)(64 * (j >> 2) + 4 * g + (j & 3)) * P + col);
+            S[j][0] = v.x; S[j][1] = v.y; S[j][2] = v.z; S[j][3] = v.w;
+        }
+    }
+    float prod = 1.0f;
+    for (int c0 = 0, buf = 0; c0 < count; c0 += CH, buf ^= 1) {
+        const int cn = min(CH, count - c0);
+        if (tid < CH) {
+            const float dt = lin ? pre_dt : seq_softplus(pre_dt + bias);
+            *reinterpret_cast<float2*>(dts + (buf * CH + tid) * 2) = make_float2(dt, lin ? pre_dec : expf(-rate * dt));
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // this wave's rows have landed
+        __syncthreads();                                                // everybody's have, and the other buffer is consumed
+        if (p.act) {                                                    // (x, B and C through SiLU in place; the decays stay)
+            const int end = (WL - VEC * N) >> 2;
+            for (int i = wave; i < cn; i += nw)
+                for (int u = lane; u < end; u += 64) {
+                    float4* at = reinterpret_cast<float4*>(lds + (size_t)(buf * CH + i) * WL) + u;
+                    const float4 v = *at;
+                    *at = make_float4(seq_silu(v.x), seq_silu(v.y), seq_silu(v.z), seq_silu(v.w));
+                }
+            __syncthreads();
+        }
+        if (c0 + CH < count) {
+            stage(c0 + CH, buf ^ 1);
+            fetch(c0 + CH);
+        }
+        const float* row = lds + (size_t)buf * CH * WL;
+        const float* dd = dts + buf * CH * 2;
+        float4 keep = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 2
+        for (int i = 0; i < cn; ++i, row += WL) {
+            const float2 sc = *reinterpret_cast<const float2*>(dd + 2 * i);
+            const float4 xv = *reinterpret_cast<const float4*>(row + col);
+            const float dx[4] = {sc.x * xv.x, sc.x * xv.y, sc.x * xv.z, sc.x * xv.w};
+            float part[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const float4 bv = *reinterpret_cast<const float4*>(row + P + 64 * q + 4 * g);
+                float4 cv = make_float4(0.f, 0.f, 0.f, 0.f), av = make_float4(sc.y, sc.y, sc.y, sc.y);
+                if constexpr (!STATE_ONLY) cv = *reinterpret_cast<const float4*>(row + P + N + 64 * q + 4 * g);
+                if constexpr (VEC) av = *reinterpret_cast<const float4*>(row + P + 2 * N + 64 * q + 4 * g);
+                const float be[4] = {bv.x, bv.y, bv.z, bv.w}, ce[4] = {cv.x, cv.y, cv.z, cv.w}, ae[4] = {av.x, av.y, av.z, av.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        S[4 * q + e][c] = fmaf(ae[e], S[4 * q + e][c], be[e] * dx[c]);
+                        if constexpr (!STATE_ONLY) part[c] = fmaf(S[4 * q + e][c], ce[e], part[c]);
+                    }
+            }
+            if constexpr (STATE_ONLY) {
+                prod *= sc.y;
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) part[c] = row16_ror<1>(row16_ror<2>(row16_ror<4>(row16_ror<8>(part[c]))));
+                if (i == g) keep = make_float4(fmaf(dskip, xv.x, part[0]), fmaf(dskip, xv.y, part[1]), fmaf(dskip, xv.z, part[2]), fmaf(dskip, xv.w, part[3]));
+            }
+        }
+        if (!STATE_ONLY && g < cn) *reinterpret_cast<float4*>(p.y + (size_t)(first + c0 + g) * inner + h * P + col) = keep;
+    }
+    if (p.mode == 2 && !last_seg) return;                               // only the portion's last segment leaves the slot's state
+    float* dst = STATE_ONLY ? p.seg_state + seg_at * N * P : st;
+#pragma unroll
+    for (int j = 0; j < 4 * Q; ++j)
+        *reinterpret_cast<float4*>(dst + (size_t)(64 * (j >> 2) + 4 * g + (j & 3)) * P + col) = make_float4(S[j][0], S[j][1], S[j][2], S[j][3]);
+    if (STATE_ONLY && tid == 0 && !VEC) p.seg_prod[seg_at] = prod;
+}
+
+// whether k_scan_rows takes the sizes and the sources' places, and its tokens per chunk (0: it does not)
+static int scan_rows_chunk(const ScanP& p) {
+    if (p.n_state % 64 || p.n_state > 256 || p.n_state == 192 || p.vdim % 16 || p.vdim > (p.n_state == 256 ? 128 : 256) || p.ones) return 0;
+    uintptr_t at = (uintptr_t)p.state | (uintptr_t)p.y | (uintptr_t)p.seg_state;
+    int64_t cols = 0;
+    if (p.kind == 1) {
+        at |= (uintptr_t)p.proj | (uintptr_t)p.decay_v;
+        cols = p.ld | p.v_col0 | p.k_col0 | p.q_col0;
+    } else {
+        at |= (uintptr_t)p.xbc;
+    }
+    if ((at & 15) || (cols & 3)) return 0;
+    const int row = p.vdim + (2 + p.vec) * p.n_state;
+    for (int ch = 16; ch >= 8; ch >>= 1)
+        if (2 * ch * (row + 2) * 4 <= 68 * 1024) return ch;
+    return 0;
+}
+
+template <int Q, bool VEC, int CH, bool STATE_ONLY>
+static int launch_scan_rows(const ScanP& p, const zls_batch_t* b, hipStream_t hs) {
+    const int lds = 2 * CH * (p.vdim + (2 + p.vec) * p.n_state + 2) * 4;
+    if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(&k_scan_rows<Q, VEC, CH, STATE_ONLY>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+        return ZL_ELIMIT;
+    hipLaunchKernelGGL((k_scan_rows<Q, VEC, CH, STATE_ONLY>), dim3((unsigned)(b->n_seq * p.n_seg), (unsigned)p.heads), dim3((unsigned)(p.vdim * 4)), lds, hs, p, *b);
+    return zl_launch_status();
+}
+template <int Q, bool VEC>
+static int launch_scan_rows(const ScanP& p, const zls_batch_t* b, int ch, hipStream_t hs) {
+    if (ch == 16) return p.mode == 1 ? launch_scan_rows<Q, VEC, 16, true>(p, b, hs) : launch_scan_rows<Q, VEC, 16, false>(p, b, hs);
+    return p.mode == 1 ? launch_scan_rows<Q, VEC, 8, true>(p, b, hs) : launch_scan_rows<Q, VEC, 8, false>(p, b, hs);
+}
+static int launch_scan_rows(const ScanP& p, const zls_batch_t* b, int ch, hipStream_t hs) {
+    if (p.vec) return p.n_state == 64 ? launch_scan_rows<1, true>(p, b, ch, hs) : p.n_state == 128 ? launch_scan_rows<2, true>(p, b, ch, hs) : launch_scan_rows<4, true>(p, b, ch, hs);
+    return p.n_state == 64 ? launch_scan_rows<1, false>(p, b, ch, hs) : p.n_state == 128 ? launch_scan_rows<2, false>(p, b, ch, hs) : launch_scan_rows<4, false>(p, b, ch, hs);
+}
+
 // vector decays: the product of a segment's decays per (sequence, segment, head, state row); the last segment needs none.  The 1024 threads
 // are (row, part of the segment's tokens): every part multiplies its tokens in order, the parts meet in LDS and are multiplied in order
 __global__ __launch_bounds__(1024) void k_seg_decay_prod(const ScanP p, const zls_batch_t b) {
@@ -337,6 +530,7 @@ static int launch_scan(ScanP& p, int64_t heads, int64_t vdim, int64_t n_state, c
     ZL_CHECK_ARG((int64_t)b->n_seq * n_seg <= 0x7fffffff, ZL_ELIMIT);
     const dim3 grid((unsigned)(b->n_seq * n_seg), (unsigned)heads, (unsigned)col_parts), block((unsigned)threads);
     hipStream_t hs = (hipStream_t)s;
+    const int wide = scan_rows_chunk(p);
     // (up to 256 threads the compiler may use the whole register file for the state and the prefetched chunk, up to 512 half of it: the
     // 32 states, 32 prefetched numbers and 64 offsets of a thread still fit without scratch memory)
 #define SCAN(NPT)                                                                                        \
@@ -344,7 +538,8 @@ static int launch_scan(ScanP& p, int64_t heads, int64_t vdim, int64_t n_state, c
     else if (threads <= 512) hipLaunchKernelGGL((k_ssm_scan<NPT, 512>), grid, block, lds, hs, p, *b);    \
     else if (threads <= 640) hipLaunchKernelGGL((k_ssm_scan<NPT, 640>), grid, block, lds, hs, p, *b);    \
     else hipLaunchKernelGGL((k_ssm_scan<NPT, 1024>), grid, block, lds, hs, p, *b);
-#define SCAN_ANY if (npt <= 8) { SCAN(8) } else if (npt <= 16) { SCAN(16) } else { SCAN(32) }
+#define SCAN_ANY if (wide) { const int rc = launch_scan_rows(p, b, wide, hs); if (rc != ZL_OK) return rc; }            \
+    else if (npt <= 8) { SCAN(8) } else if (npt <= 16) { SCAN(16) } else { SCAN(32) }
     if (!segmented) {
         p.mode = 0;
         SCAN_ANY

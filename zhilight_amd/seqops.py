@@ -381,9 +381,17 @@ SCAN_SEGMENT = 256      # tokens per segment of a long portion, at most (ssm_sca
 SCAN_WAVES = 2048       # waves that a scan of one step should bring onto the chip
 
 
-def scan_segment(n_tok, waves, longest, shortest=16):
-    """tokens per segment for a scan that runs `waves` waves per segment: as long as the step's segments together still make SCAN_WAVES waves"""
-    return max(shortest, min(longest, (n_tok * waves // SCAN_WAVES + 15) // 16 * 16))
+SCAN_ROWS_WAVES = 3072  # the same for the states of whole 64s of rows and whole 16s of columns, whose kernel holds 4 waves per SIMD (2952 tokens,
+                        # 16 heads of 128 x 128: 352 / 263 / 195 / 206 us for 1024 / 2048 / 3072 / 4096; 2048 tokens, 64 heads of 64 x 128: 232 / 229 / 212 / 226)
+
+
+def scan_segment(n_tok, waves, longest, shortest=16, fill=None):
+    """tokens per segment for a scan that runs `waves` waves per segment: as long as the step's segments together still make `fill` (SCAN_WAVES) waves"""
+    return max(shortest, min(longest, (n_tok * waves // (fill or SCAN_WAVES) + 15) // 16 * 16))
+
+
+def _scan_fill(columns, n_state):
+    return SCAN_ROWS_WAVES if n_state in (64, 128, 256) and columns % 16 == 0 else SCAN_WAVES
 
 
 def _scan_waves(heads, columns, n_state):
@@ -400,7 +408,7 @@ def ssm_scan(xbc, proj, dt_col0, dt_bias, a_log, d, state, heads, vdim, n_state,
     if xbc.shape[1] != heads * vdim + 2 * groups * n_state or tuple(state.shape[1:]) != (heads, n_state, vdim):
         raise ZLError("ssm_scan: shapes")
     y = torch.empty((batch.n_tok, heads * vdim), dtype=torch.float32, device=xbc.device)
-    seg_len = scan_segment(batch.n_tok, _scan_waves(heads, vdim, n_state), SCAN_SEGMENT) if seg_len is None else seg_len
+    seg_len = scan_segment(batch.n_tok, _scan_waves(heads, vdim, n_state), SCAN_SEGMENT, fill=_scan_fill(vdim, n_state)) if seg_len is None else seg_len
     ws = None
     if seg_len > 0 and batch.c.max_count > seg_len:
         ws = torch.empty(int(lib().zls_ssm_scan_workspace_bytes(_i(batch.n_seq), _i(batch.c.max_count), _i(seg_len), _i(heads), _i(vdim),
@@ -751,7 +759,7 @@ def decay_scan(proj, q_col0, k_col0, v_col0, act, decay_h, decay_t, gain_t, norm
         if t is not None and tuple(t.shape) != (batch.n_tok, heads):
             raise ZLError("decay_scan: per-token decays / gains are (n_tok, heads)")
     y = torch.empty((batch.n_tok, heads * P), dtype=torch.float32, device=proj.device)
-    seg_len = scan_segment(batch.n_tok, _scan_waves(heads, P, dim), SCAN_SEGMENT) if seg_len is None else seg_len
+    seg_len = scan_segment(batch.n_tok, _scan_waves(heads, P, dim), SCAN_SEGMENT, fill=_scan_fill(P, dim)) if seg_len is None else seg_len
     ws = None
     if seg_len > 0 and batch.c.max_count > seg_len:
         ws = torch.empty(int(lib().zls_ssm_scan_workspace_bytes(_i(batch.n_seq), _i(batch.c.max_count), _i(seg_len), _i(heads), _i(P), _i(dim))) // 4,
