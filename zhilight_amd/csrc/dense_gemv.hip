@@ -1,3 +1,5 @@
+// One row (and rows whose k is no whole 64s) runs k_dense_gemv, described next; 2 and more rows run zl_stream16.h.
+//
 // dense_gemv.hip -- y = T(alpha * x . W^T + bias) for small M (decode lm_head / NormalLinear), W (N,K)
 // fp16 or bf16 row-major.  SURVEY 8a row a21 (the reference calls cuBLASLt with fp32 compute:
 // bm/functions/gemm.cpp:258-344, src/nn/embedding/embedding.cu:274-289).
@@ -9,6 +11,7 @@
 // butterfly per row, no atomics / split-K.
 #include "zl_common.h"
 #include "zl_stage.h"
+#include "zl_stream16.h"
 
 namespace {
 
@@ -229,6 +232,37 @@ __global__ __launch_bounds__(64) void k_gemm_nt_f32(const uint16_t* __restrict__
     if (lane == 0) y[(int64_t)row * n + col] = alpha * acc;
 }
 
+// zl_stream16.h's results: y = T(alpha * sum + bias), and with ws the greedy candidates: a thread keeps the best of its columns (they ascend: the
+// first on ties), 16 threads hold a row; the workgroup leaves one candidate per row, slots without a workgroup stay empty
+template <int DT>
+struct SmallEpi {
+    uint16_t* y; const uint16_t* bias; float2* ws;
+    float alpha;
+    int m, n, total_waves;
+    float best_v; int best_i;
+    __device__ __forceinline__ void put(int r, int col, float v) {
+        const uint16_t y16 = ZT<DT>::from_f32(alpha * v + (bias ? ZT<DT>::to_f32(bias[col]) : 0.f));
+        y[(size_t)r * n + col] = y16;
+        const float yv = ZT<DT>::to_f32(y16);
+        if (yv > best_v || best_i == 0x7fffffff) { best_v = yv; best_i = col; }
+    }
+    __device__ __forceinline__ void finish() {
+        if (!ws) return;
+        const int r = threadIdx.x >> 4;                        // (at most 4 rows come with ws: one per 16 threads)
+#pragma unroll
+        for (int off = 1; off < 16; off <<= 1) {
+            const float ov = __shfl_xor(best_v, off, 64);
+            const int oi = __shfl_xor(best_i, off, 64);
+            if (oi != 0x7fffffff && (ov > best_v || (ov == best_v && oi < best_i) || best_i == 0x7fffffff)) { best_v = ov; best_i = oi; }
+        }
+        if (r < m && (threadIdx.x & 15) == 0) {
+            float2* row = ws + (size_t)r * total_waves;
+            row[blockIdx.x] = make_float2(best_v, __int_as_float(best_i));
+            for (int i = blockIdx.x + gridDim.x; i < total_waves; i += gridDim.x) row[i] = make_float2(0.f, __int_as_float(0x7fffffff));
+        }
+    }
+};
+
 }  // namespace
 
 static int dense_waves(int64_t n, int* rows_per_wave, int* gx) {
@@ -266,6 +300,20 @@ static int gemm_nt_small_m_impl(const uint16_t* x, int64_t ldx, const uint16_t* 
     p.total_waves = dense_waves(n, &p.rows_per_wave, &gx);
     p.argmax_ws = reinterpret_cast<float2*>(argmax_ws);
     hipStream_t hs = (hipStream_t)s;
+    // 2 and more rows: the streaming kernel; with a norm or a greedy pick up to 4 (x lies in LDS then).  One row: only narrow matrices, where its
+    // shorter ramp counts (2304 x 5760 8.3 us against 9.6; 128256 x 4096 173 against 162) -- the norm and the pick stay with k_dense_gemv
+    const bool extra = norm_weight || argmax_ws;
+    if (s16_takes(x, ldx, w, m, n, k) && (m >= 2 ? !extra || (m <= 4 && (!norm_weight || k <= 8192)) : !extra && n <= 16384)) {
+        const Stream16P g = {x, w, ldx, (int)m, (int)n, (int)k, norm_weight, norm_eps};
+#define ZL_STREAM(DT)                                                                                                                   \
+    {                                                                                                                                   \
+        const SmallEpi<DT> e = {y, bias, p.argmax_ws, alpha, (int)m, (int)n, p.total_waves, -INFINITY, 0x7fffffff};                     \
+        return norm_weight ? s16_launch_norm<DT>(g, e, hs) : s16_launch<DT>(g, e, hs);                                                  \
+    }
+        if (dtype == ZL_F16) ZL_STREAM(ZL_F16)
+        ZL_STREAM(ZL_BF16)
+#undef ZL_STREAM
+    }
 #define ZL_DISPATCH(DT)                                      \
     switch (mt) {                                            \
         case 1: return launch<DT, 1>(p, gx, gy, hs);         \

@@ -5,7 +5,8 @@
 // shape conditions.  Two kernels:
 //   k_seq_gemv  m <= 8 rows (decode steps): a wave streams the weight rows of 1 / 2 / 4 output columns (for <= 2 / 4 / 8 activation rows)
 //               once, 16-byte loads, all sums in registers, butterflies at the end -- the weight matrix is read exactly once.
-//   k_seq_gemv_mfma  3 .. 16 rows in bf16: the same streaming with the products on the matrix cores (see there).
+//   zl_stream16.h  up to 32 bf16 rows whose k comes to whole 64s: weights through LDS-DMA rings, products on the matrix cores.
+//   k_seq_gemv_mfma  3 .. 16 rows in bf16, any other k: the same streaming with the products on the matrix cores (see there).
 //   k_seq_gemm  more rows (prompt portions, mixed steps): 128 x 128 or 64 x 64 output tile per workgroup of 4 waves (2 x 2; a wave =
 //               4 x 4 or 2 x 2 MFMA tiles of 16 x 16), 32-k slices of x and W staged through LDS (zero-filled past the edges), the next slice's global
 //               loads issued before the current slice's MFMAs.  bf16: v_mfma_f32_16x16x32_bf16; fp32: v_mfma_f32_16x16x4_f32.
@@ -15,7 +16,7 @@
 // Each has instantiations with an epilogue: EPI 1 adds a bias and writes leading columns once more in the serving format, EPI 2 also applies
 // an activation and a factor looked up per row.
 #include "seq_common.h"
-#include "../csrc/zl_gemm16.h"
+#include "../csrc/zl_stream16.h"
 
 namespace {
 
@@ -456,9 +457,24 @@ void launch_tiled(const GemmP& p, hipStream_t hs) {
     }
 }
 
+template <int DT, int ODT, int EPI>
+struct StreamEpi {
+    GemmP p;
+    __device__ __forceinline__ void put(int r, int col, float v) { ::put<DT, ODT, EPI>(p, r, col, v); }
+    __device__ __forceinline__ void finish() {}
+};
+
 template <int DT, int ODT, int EPI = 0>
 int launch(const GemmP& p, hipStream_t hs) {
     if constexpr (DT == ZL_BF16) {
+        if (s16_takes(p.x, p.ldx, p.w, p.m, p.n, p.k)) {
+            const Stream16P g = {reinterpret_cast<const uint16_t*>(p.x), reinterpret_cast<const uint16_t*>(p.w), p.ldx, p.m, p.n, p.k, nullptr, 0.f};
+            return s16_launch<ZL_BF16>(g, StreamEpi<DT, ODT, EPI>{p}, hs);
+        }
+        if (!p.part && p.m > 8 && g16_takes(p.x, p.ldx, p.w, p.ldw, p.k)) {                     // (wide matrices: see s16_takes)
+            launch_tiled<DT, ODT, EPI>(p, hs);
+            return zl_launch_status();
+        }
         if (!p.part && p.m >= 3 && p.m <= 16 && p.vec && (p.k & 7) == 0) {
             hipLaunchKernelGGL((k_seq_gemv_mfma<ODT, EPI>), dim3((unsigned)((p.n + 15) / 16)), dim3(256), 0, hs, p);
             return zl_launch_status();

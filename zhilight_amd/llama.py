@@ -370,7 +370,9 @@ class NormalLinear:
             return ops.gemm_nt_small_m(x2, self.weight, bias=self.bias, out=out, norm_weight=norm_weight, norm_eps=norm_eps)
         if norm_weight is not None:
             x2 = ops.rmsnorm(x2, norm_weight, norm_eps)
-        # 5..32 rows (decode batches of the unquantised models): the ZLD16M copy of the matrix -- 1 KiB contiguous
+        if ops.streams_rows(x2.shape[0], self.dim_out, self.dim_in):
+            return ops.gemm_nt_small_m(x2, self.weight, bias=self.bias, out=out)
+        # 9..32 rows of a wide matrix (decode batches of the unquantised models): the ZLD16M copy of the matrix -- 1 KiB contiguous
         # fragment loads, 5.95 instead of 5.0 TB/s on the Llama-3 lm_head, the same bits; packed on first use outside stream capture.
         # A second copy of the weights: ZL_DENSE_PACKED=0 keeps only the row-major one
         if x2.shape[0] <= 32 and os.environ.get("ZL_DENSE_PACKED", "1") != "0":
@@ -1245,6 +1247,8 @@ class LLaMA:
             if rows > 4 and argmax_ws is None and c.dim_model % 128 == 0:
                 # more rows than the streaming GEMV takes per pass: the MFMA GEMM; up to 32 rows (decode batches) on the ZLD16M copy of
                 # the matrix -- packed on first use, OUTSIDE stream capture (run a step eagerly before capturing it, as bench.py does)
+                if ops.streams_rows(rows, *self.lm_head.shape):
+                    return ops.gemm_nt_small_m(xn, self.lm_head, out=out)
                 if rows <= 32 and os.environ.get("ZL_LM_HEAD_PACKED", "1") != "0":
                     if getattr(self, "_lm_head_m", None) is None and not torch.cuda.is_current_stream_capturing():
                         self._lm_head_m = ops.DenseMWeight(self.lm_head)

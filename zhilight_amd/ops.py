@@ -615,6 +615,12 @@ def gemm_nt_small_m(x, weight, bias=None, alpha=1.0, out=None, norm_weight=None,
     return out
 
 
+def streams_rows(m, n, k):
+    """whether gemm_nt_small_m streams a matrix once for all m rows (csrc/zl_stream16.h): decode batches; more rows of a wide matrix, or another k,
+    are better off with the packed copy or the tiles"""
+    return k % 64 == 0 and (m <= 8 or (m <= 32 and n <= 16384))
+
+
 def gemm_nt(x, weight, bias=None, alpha=1.0, out=None):
     """functions::Gemm(trans_b=True) for any M on the matrix cores (K % 128 == 0); M <= 4 callers want
     gemm_nt_small_m, which streams the weights at HBM speed."""
