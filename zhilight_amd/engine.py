@@ -89,7 +89,7 @@ class Engine:
             base += len(e.tokens)
         dev = self.model.device
         batch = seqops.RaggedBatch(seqs, self.cache.page_size, dev)
-        ids = torch.tensor(flat + rows, dtype=torch.int32).to(dev)
+        ids = seqops.to_device(flat + rows, dev)
         tokens, want = ids[:len(flat)], (ids[len(flat):] if rows else None)
         return self.model.forward(tokens, batch, want)
 

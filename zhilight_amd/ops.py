@@ -15,14 +15,14 @@ import math
 import torch
 
 from . import _lib
-from ._lib import W4Layout, W4Opts, ZLError, check, lib
+from ._lib import W4Layout, W4Opts, ZLError, check, lib, raw_stream
 
 F16, BF16 = 0, 1
 EPI_BIAS, EPI_ADD_C, EPI_RESIDUAL, EPI_SILU_MUL, EPI_SILU_MUL_F32 = 1, 2, 4, 8, 16
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return C.c_void_p(raw_stream())
 
 
 def _p(t):
@@ -343,6 +343,9 @@ _W4_ENV = (("phase_rounds", "ZL_W4_PHASE_ROUNDS"), ("phase_ksplit", "ZL_W4_PHASE
            ("tiled_bm", "ZL_W4_TILED_BM"), ("tiled_splitk", "ZL_W4_TILED_SPLITK"), ("mfma_ks", "ZL_MFMA_KS"), ("mfma_rounds", "ZL_MFMA_ROUNDS"), ("tiled_wide", "ZL_W4_TILED_WIDE"),
            ("slab", "ZL_W4_SLAB"), ("slab_min_m", "ZL_W4_SLAB_MIN_M"), ("slab_nw", "ZL_W4_SLAB_NW"), ("slab_gpw", "ZL_W4_SLAB_GPW"), ("slab_r", "ZL_W4_SLAB_R"),
            ("defer_norm", "ZL_DEFER_NORM"))
+# the environment's own dictionary where there is one (its keys are encoded): os.environ.get encodes and decodes, 26 us for these names on every launch
+_ENVIRON = getattr(os.environ, "_data", os.environ)
+_W4_NAMES = tuple(os.environ.encodekey(env) if _ENVIRON is not os.environ else env for env in [e for _, e in _W4_ENV] + ["ZL_W4_PHASE_SMALL", "ZL_W4_SMALL_ALGO"])
 
 
 def w4_scratch(device, m, n):
@@ -377,6 +380,8 @@ def _w4_opts(device, m, n):
     buf = w4_scratch(device, m, n) if m > 2 else None   # up to 2 rows no launcher splits over workgroups (3..4: the long-K slab route)
     if buf is not None:
         o.scratch, o.scratch_bytes = buf.data_ptr(), buf.numel()
+    if not any(name in _ENVIRON for name in _W4_NAMES):     # (the usual case)
+        return o
     for field, env in _W4_ENV:
         v = os.environ.get(env)
         if v:

@@ -10,7 +10,7 @@ import os
 
 import torch
 
-from ._lib import ZLError
+from ._lib import ZLError, raw_stream
 
 BF16, F32 = 1, 2
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -75,7 +75,7 @@ def check(status, what):
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return C.c_void_p(raw_stream())
 
 
 def _p(t):
@@ -108,6 +108,16 @@ def _f32(*ts):
     for t in ts:
         if t is not None and t.dtype != torch.float32:
             raise ZLError("this argument is fp32 in both modes")
+
+
+def to_device(values, device):
+    """an int32 device tensor of a list of numbers.  From page-locked memory, so that the copy queues behind the launches before it and the host goes
+    on: a copy from ordinary memory waits until the stream has drained, once or twice per step (torch keeps a block until its copy is done).
+    While a graph is captured the ordinary copy stays: it is refused there, a replay would read the block after it has gone to somebody else."""
+    device = torch.device(device)
+    if device.type == "cuda" and not torch.cuda.is_current_stream_capturing():
+        return torch.tensor(values, dtype=torch.int32, pin_memory=True).to(device, non_blocking=True)
+    return torch.tensor(values, dtype=torch.int32).to(device)
 
 
 class RaggedBatch:
@@ -145,9 +155,7 @@ class RaggedBatch:
                 for r0 in range(0, count, 64):
                     q_tiles += [starts[i] + r0, min(64, count - r0), i]
         # ONE host array, one copy: [seq_start | seq_pos0 | seq_slot | tok_seq | page_table | ctx_start | ctx_rows | q_tiles]
-        host = torch.tensor(starts + [s[1] for s in seqs] + [s[2] for s in seqs] + tok_seq + table + ctx_start + ctx_rows + q_tiles,
-                            dtype=torch.int32)
-        self.dev = host.to(device, non_blocking=False)
+        self.dev = to_device(starts + [s[1] for s in seqs] + [s[2] for s in seqs] + tok_seq + table + ctx_start + ctx_rows + q_tiles, device)
         o = [0, n_seq + 1, 2 * n_seq + 1, 3 * n_seq + 1, 3 * n_seq + 1 + starts[-1]]
         base = self.dev.data_ptr()
         self.n_seq, self.n_tok, self.starts = n_seq, starts[-1], starts
@@ -184,7 +192,7 @@ class RaggedBatch:
                 ctx_pos0.append(c0)
                 rows = [pages[j // ps] * ps + j % ps for j in range(c0, pos0 + count)]
                 ctx_rows += rows + [rows[0]] * (-len(rows) % 64)
-            dev = torch.tensor(ctx_start + ctx_pos0 + ctx_rows, dtype=torch.int32).to(self.dev.device)
+            dev = to_device(ctx_start + ctx_pos0 + ctx_rows, self.dev.device)
             n = self.n_seq
             self._windowed[window] = (dev[:n], dev[n:2 * n], dev[2 * n:], len(ctx_rows))
         return self._windowed[window]
