@@ -16,6 +16,26 @@ template <> struct SeqT<ZL_F32> {
     static __device__ __forceinline__ void st(void* p, size_t i, float v) { reinterpret_cast<float*>(p)[i] = v; }
 };
 
+// four consecutive numbers (16 / 8 aligned bytes)
+__device__ __forceinline__ float4 seq_ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+template <int DT>
+__device__ __forceinline__ float4 seq_ld4(const void* p, size_t i) {
+    if constexpr (DT == ZL_F32) return seq_ld4(reinterpret_cast<const float*>(p) + i);
+    else {
+        const uint2 u = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(p) + i);
+        return make_float4(__builtin_bit_cast(float, u.x << 16), __builtin_bit_cast(float, u.x & 0xffff0000u), __builtin_bit_cast(float, u.y << 16),
+                           __builtin_bit_cast(float, u.y & 0xffff0000u));
+    }
+}
+template <int DT>
+__device__ __forceinline__ void seq_st4(void* p, size_t i, float a, float b, float c, float d) {
+    if constexpr (DT == ZL_F32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(p) + i) = make_float4(a, b, c, d);
+    else
+        *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(p) + i) =
+            make_uint2(ZT<ZL_BF16>::from_f32(a) | (uint32_t)ZT<ZL_BF16>::from_f32(b) << 16, ZT<ZL_BF16>::from_f32(c) | (uint32_t)ZT<ZL_BF16>::from_f32(d) << 16);
+}
+static inline bool seq_aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }      // (NULL is)
+
 __device__ __forceinline__ float seq_silu(float v) { return v / (1.0f + expf(-v)); }
 __device__ __forceinline__ float seq_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
 __device__ __forceinline__ float seq_softplus(float v) { return v > 20.0f ? v : log1pf(expf(v)); }

@@ -709,6 +709,31 @@ __global__ __launch_bounds__(256) void k_head_mix_gate(const MixP p, const zls_b
     }
 }
 
+// the same for one split without mixing or turning back (portions on the matrix cores, plain heads in whole 4s): nothing meets another thread's numbers,
+// so a thread takes 4 of them straight through (2952 tokens x 16 heads of 128: 73 -> 9.5 us)
+template <int DT>
+__global__ __launch_bounds__(256) void k_head_gate_v(const MixP p) {
+    const size_t t = blockIdx.x;
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 4, h = c / p.vdim;
+    if (c >= p.heads * p.vdim) return;
+    const float2 ml = reinterpret_cast<const float2*>(p.ml)[t * p.heads + h];
+    float f = p.plain_sum ? 1.0f : 1.0f / ml.y;
+    if (p.sink && !p.plain_sum) {
+        const float sk = p.sink[h], M = fmaxf(ml.x, sk), e = expf(ml.x - M);
+        f = e / (ml.y * e + expf(sk - M));
+    }
+    float4 v = seq_ld4(p.acc + t * p.heads * p.vdim + c);
+    v = make_float4(f * v.x, f * v.y, f * v.z, f * v.w);
+    if (p.gate && p.gate_per_head) {
+        const float g = seq_sigmoid(p.gate[t * p.ldg + p.g_col0 + h]);
+        v = make_float4(v.x * g, v.y * g, v.z * g, v.w * g);
+    } else if (p.gate) {
+        const float4 g = seq_ld4(p.gate + t * p.ldg + p.g_col0 + c);
+        v = make_float4(v.x * seq_sigmoid(g.x), v.y * seq_sigmoid(g.y), v.z * seq_sigmoid(g.z), v.w * seq_sigmoid(g.w));
+    }
+    seq_st4<DT>(p.out, t * p.ldo + c, v.x * p.out_scale, v.y * p.out_scale, v.z * p.out_scale, v.w * p.out_scale);
+}
+
 }  // namespace
 
 extern "C" int zls_rope_norm_store(float* proj, int64_t ld, int64_t q_col0, int64_t k_col0, int64_t v_col0, int64_t heads, int64_t kv_heads,
@@ -831,6 +856,14 @@ extern "C" int zls_head_mix_gate(const float* acc, const float* ml, int64_t n_sp
     p.acc = acc; p.ml = ml; p.n_splits = (int)n_splits; p.talk = talk; p.v_freq = v_freq; p.gate = gate; p.ldg = ldg; p.g_col0 = (int)g_col0;
     p.heads = (int)heads; p.kv_heads = (int)kv_heads; p.vdim = (int)vdim; p.out = out; p.sink = sink;
     p.plain_sum = plain_sum ? 1 : 0; p.gate_per_head = gate_per_head ? 1 : 0; p.ldo = ldo; p.out_scale = out_scale;
+    if (n_splits == 1 && !talk && !v_freq && heads * vdim < (1 << 26) && vdim % 4 == 0 && ldo % 4 == 0 && seq_aligned(acc) && ((uintptr_t)ml & 7) == 0 && seq_aligned(out) &&
+        (!gate || gate_per_head || (seq_aligned(gate) && ldg % 4 == 0 && g_col0 % 4 == 0))) {
+        const unsigned threads = heads * vdim > 768 ? 256 : (unsigned)((heads * vdim + 255) / 256 * 64);
+#define CALL(DT) hipLaunchKernelGGL((k_head_gate_v<DT>), dim3(b->n_tok, (unsigned)((heads * vdim + 1023) / 1024)), dim3(threads), 0, (hipStream_t)s, p);
+        ZLS_DISPATCH(dtype, CALL)
+#undef CALL
+        return zl_launch_status();
+    }
 #define CALL(DT) hipLaunchKernelGGL((k_head_mix_gate<DT>), dim3(b->n_tok, (unsigned)kv_heads), dim3(256), lds, (hipStream_t)s, p, *b);
     ZLS_DISPATCH(dtype, CALL)
 #undef CALL
