@@ -713,6 +713,14 @@ int zl_int8_gemm_nt(const int8_t* a /* (M,K) */, const int8_t* b /* (N,K) */, in
  * act is -1 without b2. */
 int zl_int8_linear(const int8_t* a, const float* sx, const int8_t* b, const uint16_t* sy, const int8_t* b2, const uint16_t* sy2,
                    const uint16_t* addend, uint16_t* out, int64_t m, int64_t n, int64_t k, float scale, int act, int dtype, zl_stream_t s);
+/* a fp16 / bf16 linear and what follows it in one launch, the bits of the separate calls:
+ *   w2 == NULL   y = T(x . w^T + bias), with `addend` (y may alias it) zl_element_add_scale(addend, that, scale, scale_residual)
+ *   w2           zl_gate_mul of T(x . w^T + bias) and T(x . w2^T + bias2), n rows each; act 0 silu, 1 gelu (act is -1 without w2)
+ * norm_weight (nullable): x is RMS-normalised first (m <= 4 and k <= 8192).  m <= 8, m > 32, or up to 16384 rows of w and w2 together;
+ * k % 64 == 0; ldx % 8 == 0; x, w and w2 16-byte aligned; otherwise ZL_ESHAPE. */
+int zl_dense_linear(const uint16_t* x, int64_t ldx, const uint16_t* w, const uint16_t* w2, const uint16_t* bias, const uint16_t* bias2,
+                    const uint16_t* addend, uint16_t* y, int64_t m, int64_t n, int64_t k, float scale, int scale_residual, int act,
+                    const uint16_t* norm_weight, float norm_eps, int dtype, zl_stream_t s);
 int zl_quant_scale_back(const int32_t* c, const float* scale_x, const uint16_t* scale_y, uint16_t* out,
                         int64_t m, int64_t n, int dtype, zl_stream_t s);
 int zl_quant_back_act_mul(const int32_t* a, const float* a_sx, const uint16_t* a_sy, const int32_t* b,

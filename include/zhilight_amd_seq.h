@@ -56,6 +56,11 @@ typedef struct {
 } zls_row_factor_t;
 int zls_gemm_nt_act(const void* x, int64_t ldx, const void* w, const float* bias, int act, void* y, int64_t ldy, void* y2, int64_t ldy2, int64_t n2,
                     const zls_row_factor_t* factor, int64_t m, int64_t n, int64_t k, float* part, int64_t n_parts, int dtype, int out_dtype, zl_stream_t s);
+/* A gated feed-forward's first product with its activation: w (2 ff, k) = gate rows, then up rows; y (m, ff) = act(x . gate^T + bias[:ff],
+ * x . up^T + bias[ff:]) as zls_act_mul computes it (act, alpha, limit: the same) from fp32 sums.  x, w and y bf16; k % 64 == 0, ldx % 8 == 0,
+ * x and w 16-byte aligned, otherwise ZL_ESHAPE. */
+int zls_gemm_nt_gated(const void* x, int64_t ldx, const void* w, const float* bias, int act, float alpha, float limit, void* y, int64_t ldy, int64_t m,
+                      int64_t ff, int64_t k, zl_stream_t s);
 /* The same with gathered rows: row r of x is x[x_rows[r]], row c of w is w[w_rows[c]] (device int32 arrays, NULL: in order; ldw: row
  * stride of w).  Always the tiled kernel.  The up-projection of cached rows that lie scattered over pages. */
 int zls_gemm_nt_gather(const void* x, int64_t ldx, const int32_t* x_rows, const void* w, int64_t ldw, const int32_t* w_rows, void* y,

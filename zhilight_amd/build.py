@@ -94,7 +94,7 @@ def build_seq(force=False, verbose=False):
     A library of its own: a checkout that serves only such a model compiles these few files and nothing of the quantised decode path."""
     srcs = sorted(os.path.join(CSRC_SEQ, f) for f in os.listdir(CSRC_SEQ) if f.endswith(".hip"))
     deps = [os.path.join(CSRC_SEQ, f) for f in os.listdir(CSRC_SEQ) if f.endswith(".h")]
-    deps += [os.path.join(CSRC, "zl_common.h"), os.path.join(CSRC, "zl_gemm16.h"), os.path.join(CSRC, "zl_stream16.h"), os.path.join(HERE, "..", "include", "zhilight_amd.h"),
+    deps += [os.path.join(CSRC, "zl_common.h"), os.path.join(CSRC, "zl_gemm16.h"), os.path.join(CSRC, "zl_stream16.h"), os.path.join(CSRC, "zl_t_ops.h"), os.path.join(HERE, "..", "include", "zhilight_amd.h"),
              os.path.join(HERE, "..", "include", "zhilight_amd_seq.h")]
     objdir = os.path.join(HERE, "build", "seq")
     os.makedirs(objdir, exist_ok=True)

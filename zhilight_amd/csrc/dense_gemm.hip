@@ -15,6 +15,8 @@
 #include <stdlib.h>
 #include "zl_common.h"
 #include "zl_gemm16.h"
+#include "zl_stream16.h"
+#include "zl_t_ops.h"
 
 namespace {
 
@@ -197,7 +199,93 @@ struct DenseEpi {
     }
 };
 
+// zl_dense_linear's results, step by step what the separate launches compute (the same bits): T(sum + bias), then the residual in T arithmetic,
+// or act(gate) * up of two such products.  What bounds it: the product; the elementwise passes over (m, n) and their launches are what goes
+// away (bf16 layers of 2304 with 5760 between: 777 rows, products + passes 202 -> 136 us; 4 rows 39 -> 31 us, five launches fewer).
+template <int DT>
+struct LinearEpi {
+    uint16_t* y; const uint16_t* bias; const uint16_t* bias2; const uint16_t* addend;
+    int n, act, scale_residual, vec;
+    uint16_t scale;
+    __device__ __forceinline__ uint16_t one(const uint16_t* b, int c, float v) const { return ZT<DT>::from_f32(v + (b ? ZT<DT>::to_f32(b[c]) : 0.f)); }
+    __device__ __forceinline__ uint16_t add(uint16_t a, uint16_t h) const {
+        return scale_residual ? t_mul<DT>(t_add<DT>(a, h), scale) : t_add<DT>(a, t_mul<DT>(h, scale));
+    }
+    __device__ __forceinline__ void put(int r, int c, float v) const {
+        const size_t at = (size_t)r * n + c;
+        const uint16_t h = one(bias, c, v);
+        y[at] = addend ? add(addend[at], h) : h;
+    }
+    __device__ __forceinline__ void put2(int r, int c, float g, float u) const { y[(size_t)r * n + c] = t_gate<DT>(one(bias, c, g), one(bias2, c, u), act); }
+    __device__ __forceinline__ void finish() const {}
+};
+template <int DT, bool GATED>
+struct LinearTileEpi {
+    LinearEpi<DT> e;
+    template <int NI, class F>
+    __device__ __forceinline__ void row(int r, int c0, int, F sum) const {
+#pragma unroll
+        for (int j = 0; j < NI; j += GATED ? 2 : 1) {
+            const int cp = c0 + 16 * j, c = GATED ? (cp >> 5) * 16 + (cp & 15) : cp;      // (GATED: cp counts the paired blocks)
+            if (c >= e.n) continue;
+            const g16_f4 v = sum(j), u = sum(GATED ? j + 1 : j);
+            if (e.vec) {                                       // (n in whole 4s: all four columns are there)
+                const size_t at = (size_t)r * e.n + c;
+                uint16_t o[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint16_t h = e.one(e.bias, c + k, v[k]);
+                    if constexpr (GATED) o[k] = t_gate<DT>(h, e.one(e.bias2, c + k, u[k]), e.act);
+                    else o[k] = h;
+                }
+                if (!GATED && e.addend) {
+                    const uint2 a = *reinterpret_cast<const uint2*>(e.addend + at);
+                    const uint16_t av[4] = {(uint16_t)(a.x & 0xffffu), (uint16_t)(a.x >> 16), (uint16_t)(a.y & 0xffffu), (uint16_t)(a.y >> 16)};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) o[k] = e.add(av[k], o[k]);
+                }
+                *reinterpret_cast<uint2*>(e.y + at) = make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if (c + k >= e.n) continue;
+                    if constexpr (GATED) e.put2(r, c + k, v[k], u[k]);
+                    else e.put(r, c + k, v[k]);
+                }
+            }
+        }
+    }
+};
+
+template <int DT>
+int dense_linear(const Stream16P& sp, const LinearEpi<DT>& e, hipStream_t hs) {
+    if (sp.m <= 32) {
+        if (sp.norm_w) return sp.w2 ? s16_launch_norm<DT, true>(sp, e, hs) : s16_launch_norm<DT>(sp, e, hs);
+        return sp.w2 ? s16_launch<DT, true>(sp, e, hs) : s16_launch<DT>(sp, e, hs);
+    }
+    const Gemm16P g = {sp.x, sp.w, sp.ldx, sp.k, sp.m, sp.w2 ? (sp.n + 15) / 16 * 32 : sp.n, sp.k, 0, 0, sp.k, sp.w2, sp.n};
+    return sp.w2 ? g16_launch<DT, true>(g, LinearTileEpi<DT, true>{e}, hs) : g16_launch<DT>(g, LinearTileEpi<DT, false>{e}, hs);
+}
+
 }  // namespace
+
+// a linear with what follows it (see zhilight_amd.h)
+extern "C" int zl_dense_linear(const uint16_t* x, int64_t ldx, const uint16_t* w, const uint16_t* w2, const uint16_t* bias, const uint16_t* bias2,
+                               const uint16_t* addend, uint16_t* y, int64_t m, int64_t n, int64_t k, float scale, int scale_residual, int act,
+                               const uint16_t* norm_weight, float norm_eps, int dtype, zl_stream_t s) {
+    ZL_CHECK_ARG(x && w && y && m > 0 && n > 0 && k > 0, ZL_EINVAL);
+    ZL_CHECK_ARG(w2 ? (act == 0 || act == 1) && !addend : act == -1 && !bias2, ZL_EINVAL);
+    ZL_CHECK_ARG(dtype == ZL_F16 || dtype == ZL_BF16, ZL_EDTYPE);
+    ZL_CHECK_ARG(ldx >= k && (!norm_weight || (m <= 4 && k <= 8192)) && m < (1 << 30) && n < (1 << 29) && ((uintptr_t)w2 & 15) == 0, ZL_ESHAPE);
+    ZL_CHECK_ARG(m <= 32 ? s16_takes(x, ldx, w, m, w2 ? 2 * n : n, k) : g16_takes(x, ldx, w, k, k), ZL_ESHAPE);
+    const Stream16P p = {x, w, ldx, (int)m, (int)n, (int)k, norm_weight, norm_eps, w2};
+    const int vec = n % 4 == 0 && ((uintptr_t)y & 7) == 0 && ((uintptr_t)addend & 7) == 0;
+    if (dtype == ZL_F16)
+        return dense_linear<ZL_F16>(p, LinearEpi<ZL_F16>{y, bias, bias2, addend, (int)n, act, scale_residual, vec, __builtin_bit_cast(uint16_t, (_Float16)scale)}, (hipStream_t)s);
+    uint32_t u = __builtin_bit_cast(uint32_t, scale);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return dense_linear<ZL_BF16>(p, LinearEpi<ZL_BF16>{y, bias, bias2, addend, (int)n, act, scale_residual, vec, (uint16_t)(u >> 16)}, (hipStream_t)s);
+}
 
 extern "C" int64_t zl_dense_m_bytes(int64_t n, int64_t k) {
     if (n <= 0 || k <= 0 || k % 128 != 0) return ZL_ESHAPE;

@@ -304,7 +304,7 @@ static int gemm_nt_small_m_impl(const uint16_t* x, int64_t ldx, const uint16_t* 
     // shorter ramp counts (2304 x 5760 8.3 us against 9.6; 128256 x 4096 173 against 162) -- the norm and the pick stay with k_dense_gemv
     const bool extra = norm_weight || argmax_ws;
     if (s16_takes(x, ldx, w, m, n, k) && (m >= 2 ? !extra || (m <= 4 && (!norm_weight || k <= 8192)) : !extra && n <= 16384)) {
-        const Stream16P g = {x, w, ldx, (int)m, (int)n, (int)k, norm_weight, norm_eps};
+        const Stream16P g = {x, w, ldx, (int)m, (int)n, (int)k, norm_weight, norm_eps, nullptr};
 #define ZL_STREAM(DT)                                                                                                                   \
     {                                                                                                                                   \
         const SmallEpi<DT> e = {y, bias, p.argmax_ws, alpha, (int)m, (int)n, p.total_waves, -INFINITY, 0x7fffffff};                     \

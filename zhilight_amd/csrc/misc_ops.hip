@@ -4,6 +4,7 @@
 // points as the reference kernels cited at each launcher.
 #include <mutex>
 #include "zl_common.h"
+#include "zl_t_ops.h"
 
 namespace {
 
@@ -369,16 +370,6 @@ __global__ void k_rope_scatter_decode(const float* __restrict__ cosv, const floa
 // element-wise.  src/nn/block/block_kernel.cu:8-17, src/nn/linear/activation_kernel.cu:59-80
 // ------------------------------------------------------------------------------------------------
 template <int DT>
-__device__ __forceinline__ uint16_t t_add(uint16_t a, uint16_t b) {  // one rounding to T (exact sum in fp32*)
-    // fp16: the fp32 sum of two halfs is exact; bf16: may round in fp32 first (documented)
-    return ZT<DT>::from_f32(ZT<DT>::to_f32(a) + ZT<DT>::to_f32(b));
-}
-template <int DT>
-__device__ __forceinline__ uint16_t t_mul(uint16_t a, uint16_t b) {  // product of two T is exact in fp32
-    return ZT<DT>::from_f32(ZT<DT>::to_f32(a) * ZT<DT>::to_f32(b));
-}
-
-template <int DT>
 __global__ void k_add_scale(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
                             int64_t n, uint16_t scale_t, int scale_residual) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
@@ -389,11 +380,7 @@ template <int DT>
 __global__ void k_gate_mul(const uint16_t* __restrict__ g, const uint16_t* __restrict__ u, uint16_t* __restrict__ out,
                            int64_t n, int act) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const float x = ZT<DT>::to_f32(g[i]);
-        float a;
-        if (act == 0) a = x / (1.0f + expf(-x));
-        else a = 0.5f * x * (1.0f + tanhf(0.7978845608028654f * x * (1.0f + 0.044715f * x * x)));
-        out[i] = ZT<DT>::from_f32(a * ZT<DT>::to_f32(u[i]));
+        out[i] = t_gate<DT>(g[i], u[i], act);
     }
 }
 
@@ -404,11 +391,7 @@ __global__ void k_gate_fuse(const uint16_t* __restrict__ in, uint16_t* __restric
     const int64_t n = rows * ff;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t r = i / ff, j = i - r * ff;
-        const float x = ZT<DT>::to_f32(in[r * 2 * ff + j]);
-        float a;
-        if (act == 0) a = x / (1.0f + expf(-x));
-        else a = 0.5f * x * (1.0f + tanhf(0.7978845608028654f * x * (1.0f + 0.044715f * x * x)));
-        out[i] = ZT<DT>::from_f32(a * ZT<DT>::to_f32(in[r * 2 * ff + ff + j]));
+        out[i] = t_gate<DT>(in[r * 2 * ff + j], in[r * 2 * ff + ff + j], act);
     }
 }
 

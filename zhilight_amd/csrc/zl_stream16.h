@@ -17,11 +17,13 @@ struct Stream16P {
     int64_t ldx;
     int m, n, k;                                               // k % 64 == 0, rows of w are k numbers
     const uint16_t* norm_w; float norm_eps;                    // XS: nullable
+    const uint16_t* w2;                                        // DUAL: a second matrix of n rows (gate and up rows of the same outputs)
 };
 
 constexpr int s16_xrow(int k) { return k * 2 + 64; }           // bytes of a row of x in LDS (XS): rows start 16 banks apart
 
-template <int DT, int MR, int W, int D, bool XS, class Epi>
+// DUAL: a tile is 8 rows of w and the same 8 of w2, one load each; the two results of an output meet by a lane exchange
+template <int DT, int MR, int W, int D, bool XS, bool DUAL, class Epi>
 __global__ __launch_bounds__(64 * W) void k_stream16(const Stream16P p, Epi epi) {
     constexpr int kSlot = 2048 + (XS ? 0 : MR * 128), NL = 2 + (XS ? 0 : MR / 8), NB = (MR + 15) / 16;      // a slice's bytes and loads; blocks of 16 rows of x
     static_assert(XS ? MR <= 16 : MR % 8 == 0, "a load fills 8 rows");
@@ -29,7 +31,8 @@ __global__ __launch_bounds__(64 * W) void k_stream16(const Stream16P p, Epi epi)
     float* red = reinterpret_cast<float*>(s16_smem + W * D * kSlot);                                        // [2][W][MR rows of x, whole 16s][17]
     unsigned char* xs = s16_smem + W * D * kSlot + 2 * W * NB * 16 * 17 * 4;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nrow = lane & 15, kq = lane >> 4;
-    const int tiles = (p.n + 15) >> 4, S = p.k >> 6, Sw = (S - wave + W - 1) / W;                           // slices of this wave per tile
+    constexpr int TC = DUAL ? 8 : 16;                          // outputs of a tile
+    const int tiles = (p.n + TC - 1) / TC, S = p.k >> 6, Sw = (S - wave + W - 1) / W;                           // slices of this wave per tile
     const int first = blockIdx.x, step = gridDim.x, mine = (tiles - first + step - 1) / step;
     const int total = mine * Sw;                                                                            // this wave's slices, all tiles
     // a load fills 8 rows of 128 bytes: lane l -> row l / 8, unit l % 8, which holds unit (l % 8) ^ (row / 2 % 8) of the slice
@@ -41,13 +44,13 @@ __global__ __launch_bounds__(64 * W) void k_stream16(const Stream16P p, Epi epi)
     const u32x4 rx = g16_rsrc(p.x);
     int i_tile = first, i_s = wave, issued = 0;
     auto issue = [&]() {                                       // the wave's next slice into slot issued % D
-        const int c0 = i_tile * 16;
-        const u32x4 rw = g16_rsrc(p.w + (size_t)c0 * p.k);
+        const int c0 = i_tile * TC;
+        const u32x4 rw = g16_rsrc(p.w + (size_t)c0 * p.k), rw2 = DUAL ? g16_rsrc(p.w2 + (size_t)c0 * p.k) : rw;
         const uint32_t at = lds0 + (uint32_t)(issued % D) * kSlot;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int r = lr + 8 * i;
-            g16_dma(rw, (uint32_t)(min(r, p.n - 1 - c0) * p.k * 2 + ((lu ^ ((r >> 1) & 7)) * 16)), (uint32_t)i_s * 128, at + i * 1024);
+            g16_dma(i ? rw2 : rw, (uint32_t)(min(DUAL ? lr : r, p.n - 1 - c0) * p.k * 2 + ((lu ^ ((r >> 1) & 7)) * 16)), (uint32_t)i_s * 128, at + i * 1024);
         }
         if constexpr (!XS) {
 #pragma unroll
@@ -125,13 +128,16 @@ __global__ __launch_bounds__(64 * W) void k_stream16(const Stream16P p, Epi epi)
 #pragma unroll
             for (int r = 0; r < 4; ++r) rd[((wave * NB + b) * 16 + nrow) * 17 + 4 * kq + r] = acc[b][r];      // row 16 b + nrow of x, column 4 kq + r
         __syncthreads();
-        const int col = (first + t * step) * 16 + (threadIdx.x & 15);
+        const int col = (first + t * step) * TC + (threadIdx.x & (TC - 1));
 #pragma unroll
         for (int m = threadIdx.x >> 4; m < MR; m += 4 * W) {
             float v = 0.f;
 #pragma unroll
             for (int u = 0; u < W; ++u) v += rd[(u * NB * 16 + m) * 17 + (threadIdx.x & 15)];
-            if (m < p.m && col < p.n) epi.put(m, col, v);
+            if constexpr (DUAL) {
+                const float u = __shfl_xor(v, 8, 64);          // (a wave's rows m are all below MR or none)
+                if (m < p.m && col < p.n && !(threadIdx.x & 8)) epi.put2(m, col, v, u);
+            } else if (m < p.m && col < p.n) epi.put(m, col, v);
         }
     }
     epi.finish();
@@ -145,27 +151,27 @@ static inline bool s16_takes(const void* x, int64_t ldx, const void* w, int64_t 
            (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
 }
 
-template <int DT, int MR, int W, int D, bool XS, class Epi>
+template <int DT, int MR, int W, int D, bool XS, bool DUAL, class Epi>
 int s16_launch_as(const Stream16P& p, const Epi& e, int grid, hipStream_t s) {
     const int lds = W * D * (2048 + (XS ? 0 : MR * 128)) + 2 * W * ((MR + 15) / 16) * 16 * 17 * 4 + (XS ? MR * s16_xrow(p.k) : 0);
     if (lds > 64 * 1024 &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_stream16<DT, MR, W, D, XS, Epi>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_stream16<DT, MR, W, D, XS, DUAL, Epi>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
         return ZL_ELIMIT;
-    hipLaunchKernelGGL((k_stream16<DT, MR, W, D, XS, Epi>), dim3((unsigned)grid), dim3(64 * W), lds, s, p, e);
+    hipLaunchKernelGGL((k_stream16<DT, MR, W, D, XS, DUAL, Epi>), dim3((unsigned)grid), dim3(64 * W), lds, s, p, e);
     return zl_launch_status();
 }
 
 // 8 waves to a tile: with few tiles every wave's ring counts, with many one workgroup per CU walks them (256 workgroups: within 2 % of more)
-template <int DT, class Epi>
+template <int DT, bool DUAL = false, class Epi>
 int s16_launch(const Stream16P& p, const Epi& e, hipStream_t s) {
-    const int tiles = (p.n + 15) / 16, grid = tiles < 256 ? tiles : 256;
-    if (p.m <= 8) return s16_launch_as<DT, 8, 8, 3, false>(p, e, grid, s);
-    if (p.m <= 16) return s16_launch_as<DT, 16, 8, 3, false>(p, e, grid, s);
-    return s16_launch_as<DT, 32, 8, 2, false>(p, e, grid, s);
+    const int tiles = DUAL ? (p.n + 7) / 8 : (p.n + 15) / 16, grid = tiles < 256 ? tiles : 256;
+    if (p.m <= 8) return s16_launch_as<DT, 8, 8, 3, false, DUAL>(p, e, grid, s);
+    if (p.m <= 16) return s16_launch_as<DT, 16, 8, 3, false, DUAL>(p, e, grid, s);
+    return s16_launch_as<DT, 32, 8, 2, false, DUAL>(p, e, grid, s);
 }
 // up to 4 rows, normalised on the way in
-template <int DT, class Epi>
+template <int DT, bool DUAL = false, class Epi>
 int s16_launch_norm(const Stream16P& p, const Epi& e, hipStream_t s) {
-    const int tiles = (p.n + 15) / 16, grid = tiles < 256 ? tiles : 256;
-    return s16_launch_as<DT, 4, 8, 3, true>(p, e, grid, s);
+    const int tiles = DUAL ? (p.n + 7) / 8 : (p.n + 15) / 16, grid = tiles < 256 ? tiles : 256;
+    return s16_launch_as<DT, 4, 8, 3, true, DUAL>(p, e, grid, s);
 }

@@ -430,14 +430,28 @@ class DenseEncoderLayer:
         rs = self.cfg.residual_scale
         ops.element_add_scale(hidden, sub, rs, scale_residual=(self.cfg.scale_depth <= 0), out=hidden)
 
+    def _add_product(self, hidden, lin, x):
+        """hidden += lin(x) in place, in one launch where the product's kernel takes its rows"""
+        x = x.reshape(-1, x.shape[-1])
+        if hidden.dim() == 2 and hidden.is_contiguous() and ops.dense_linear_ok(x, lin.weight):
+            ops.dense_linear(x, lin.weight, lin.bias, addend=hidden, scale=self.cfg.residual_scale, scale_residual=(self.cfg.scale_depth <= 0), out=hidden)
+        else:
+            self._add(hidden, lin.forward(x))
+
     def attn_out_add(self, attn, hidden):
-        self._add(hidden, self.attn_out.forward(attn))
+        self._add_product(hidden, self.attn_out, attn)
 
     def ff_add(self, hidden, eps, act_buf=None):
-        xn = ops.rmsnorm(hidden, self.ln_ff, eps)
-        gate = self.w_in.forward(xn, out=act_buf)
-        act = ops.gate_mul(gate, self.w_gated.forward(xn), "gelu" if self.cfg.activate_fn.startswith("gelu") else "silu")
-        self._add(hidden, self.w_out.forward(act))
+        kind = "gelu" if self.cfg.activate_fn.startswith("gelu") else "silu"
+        if hidden.dim() == 2 and ops.dense_linear_ok(hidden, self.w_in.weight, self.w_gated.weight):
+            few = hidden.shape[0] <= 4 and self.w_in.dim_in <= 8192                       # (the norm rides in the product)
+            x = hidden if few else ops.rmsnorm(hidden, self.ln_ff, eps)
+            act = ops.dense_linear(x, self.w_in.weight, self.w_in.bias, up=self.w_gated.weight, up_bias=self.w_gated.bias, act=kind,
+                                   norm_weight=self.ln_ff if few else None, norm_eps=eps, out=act_buf)
+        else:
+            xn = ops.rmsnorm(hidden, self.ln_ff, eps)
+            act = ops.gate_mul(self.w_in.forward(xn, out=act_buf), self.w_gated.forward(xn), kind)
+        self._add_product(hidden, self.w_out, act)
 
 
 class Int8Linear:

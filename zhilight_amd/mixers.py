@@ -1016,7 +1016,7 @@ class GatedFF:
         return sum(t.numel() * t.element_size() for t in (self.w_gu, self.w_down))
 
     def forward(self, h):
-        return seqops.gemm_nt(seqops.act_mul(seqops.gemm_nt(h, self.w_gu, bias=self.in_bias), h.dtype, kind=self.act), self.w_down, bias=self.out_bias)
+        return seqops.gemm_nt(seqops.gated_product(h, self.w_gu, self.act, self.in_bias), self.w_down, bias=self.out_bias)
 
     def bind(self, cache, dtype):
         pass

@@ -626,6 +626,36 @@ def streams_rows(m, n, k):
     return k % 64 == 0 and (m <= 8 or (m <= 32 and n <= 16384))
 
 
+def dense_linear_ok(x, weight, up=None):
+    """whether dense_linear takes the product (prompt chunks and decode batches of rows in whole 64s)"""
+    n = weight.shape[0] * (1 if up is None else 2)
+    return (weight.shape[1] % 64 == 0 and weight.shape[1] <= 1 << 22 and (x.shape[0] > 32 or streams_rows(x.shape[0], n, weight.shape[1])) and x.is_contiguous()
+            and (x.data_ptr() | weight.data_ptr() | (0 if up is None else up.data_ptr())) % 16 == 0)
+
+
+def dense_linear(x, weight, bias=None, addend=None, scale=1.0, scale_residual=True, up=None, up_bias=None, act="silu", norm_weight=None, norm_eps=1e-5,
+                 out=None):
+    """a linear and what follows it in one launch, the bits of the separate calls: gemm_nt, with `addend` element_add_scale(addend, .) (out may be the
+    addend), with `up` gate_mul of both products; norm_weight (up to 4 rows of at most 8192): rmsnorm first.  See dense_linear_ok."""
+    _chk_cuda(x, weight, bias, addend, up, up_bias, norm_weight)
+    m, k = x.shape
+    n = weight.shape[0]
+    if weight.shape[1] != k or (up is not None and up.shape != weight.shape):
+        raise ZLError("size K mismatch")
+    if addend is not None and tuple(addend.shape) != (m, n):
+        raise ZLError("a,b shape mismatch")
+    if act not in ("silu", "gelu"):
+        raise ZLError("Unsupported gate type: " + act)
+    if out is None:
+        out = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    else:
+        _chk_out(out, m, n, x.dtype, x.device, "dense_linear")
+    check(lib().zl_dense_linear(_p(x), _i(x.stride(0)), _p(weight), _p(up), _p(bias), _p(up_bias), _p(addend), _p(out), _i(m), _i(n), _i(k), _f(scale),
+                                C.c_int(int(scale_residual)), C.c_int(-1 if up is None else 0 if act == "silu" else 1), _p(norm_weight), _f(norm_eps),
+                                C.c_int(_dt(x)), _stream()), "dense_linear")
+    return out
+
+
 def gemm_nt(x, weight, bias=None, alpha=1.0, out=None):
     """functions::Gemm(trans_b=True) for any M on the matrix cores (K % 128 == 0); M <= 4 callers want
     gemm_nt_small_m, which streams the weights at HBM speed."""

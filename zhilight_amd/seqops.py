@@ -20,7 +20,7 @@ SYMBOLS = ["zls_version", "zls_gemm_nt", "zls_gemm_nt_act", "zls_embed", "zls_to
            "zls_conv_silu", "zls_ssm_scan", "zls_ssm_scan_workspace_bytes", "zls_selective_scan", "zls_selective_scan_workspace_bytes", "zls_gated_group_norm", "zls_layer_norm",
            "zls_add_layer_norm", "zls_rope_norm_store", "zls_window_attention", "zls_window_attention_prompt", "zls_head_mix_gate", "zls_decay_scan", "zls_exp_gates",
            "zls_linear_attn_finish", "zls_moe_route", "zls_moe_align", "zls_gemm_nt_grouped", "zls_silu_mul", "zls_moe_combine", "zls_rms_norm",
-           "zls_add_rms_norm", "zls_scale_softcap", "zls_act_mul", "zls_short_conv", "zls_lowrank_decay", "zls_latent_rope_store",
+           "zls_add_rms_norm", "zls_scale_softcap", "zls_act_mul", "zls_gemm_nt_gated", "zls_short_conv", "zls_lowrank_decay", "zls_latent_rope_store",
            "zls_streams_norm", "zls_streams_update", "zls_unary_act", "zls_add_branches", "zls_tanh_norm", "zls_delta_prep", "zls_delta_scan"]
 _STATUS = {-1: "invalid argument (null pointer / non-positive size)", -2: "shape not supported", -3: "dtype not supported",
            -4: "exceeds a hardware limit"}
@@ -237,6 +237,24 @@ def gemm_nt(x, w, out=None, out_dtype=torch.float32, bias=None, act=None, lead=0
     check(lib().zls_gemm_nt_act(_p(x), _i(x.stride(0)), _p(w), _p(bias), C.c_int(-1 if act is None else UNARY_ACTS[act]), _p(out), _i(n), _p(y2),
                                 _i(lead), _i(lead), f, _i(m), _i(n), _i(k), _p(part), _i(parts), C.c_int(dt_code(x.dtype)), C.c_int(dt_code(out.dtype)), _stream()), "gemm_nt")
     return (out, y2) if lead > 0 else out
+
+
+def gated_product(x, w_gu, kind="silu", bias=None):
+    """act_mul(gemm_nt(x, w_gu, bias=bias), x.dtype, kind): in one launch, with the same bits, where one workgroup per tile does all of k"""
+    m, k = x.shape
+    ff = w_gu.shape[0] // 2
+    whole = m <= 8 or (m <= 32 and 2 * ff <= 16384) or _k_parts(m, 2 * ff, k) == 1
+    if not (x.dtype == torch.bfloat16 and x.is_cuda and k % 64 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) <= 1 << 22 and whole
+            and (x.data_ptr() | w_gu.data_ptr()) % 16 == 0):
+        return act_mul(gemm_nt(x, w_gu, bias=bias), x.dtype, kind=kind)
+    _cuda(w_gu, bias)
+    _f32(bias)
+    if w_gu.shape[1] != k or w_gu.dtype != x.dtype or (bias is not None and bias.numel() != 2 * ff):
+        raise ZLError("gated_product: sizes / dtype mismatch")
+    out = torch.empty((m, ff), dtype=x.dtype, device=x.device)
+    check(lib().zls_gemm_nt_gated(_p(x), _i(x.stride(0)), _p(w_gu), _p(bias), C.c_int(ACT_KINDS[kind]), _f(1.0), _f(0.0), _p(out), _i(ff), _i(m), _i(ff), _i(k),
+                                  _stream()), "gated_product")
+    return out
 
 
 def embed(tokens, table, pos_table, scale, batch, out=None):
