@@ -14,7 +14,7 @@ def _rand(*shape, g, dtype=torch.float32, scale=1.0):
 # every block of rows of the streaming kernel, tiles of 8 and 16 outputs with ragged ends, more tiles than workgroups; each tile shape of the large
 # products, whole and ragged
 SIZES = [(1, 16, 64), (2, 7, 128), (3, 2304, 320), (4, 4100, 128), (8, 1000, 1088), (9, 50, 512), (16, 4097, 192), (32, 129, 2304), (33, 64, 64), (77, 201, 1088),
-         (257, 513, 64), (385, 1000, 64), (777, 5760, 128), (1024, 6144, 128), (2100, 4104, 64)]
+         (257, 513, 64), (385, 1000, 64), (777, 5760, 128), (565, 10750, 64), (565, 4096, 128), (1024, 6144, 128), (2100, 4104, 64)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

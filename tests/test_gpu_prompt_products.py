@@ -25,9 +25,11 @@ def _check(y, x, w, extra=0.0):
     assert bool((off <= bound).all()), float((off / bound).max())
 
 
-# 256 x 256, 256 x 128, 128 x 128 in rounds, 128 x 128 alone, 128 x 64 and 64 x 64 tiles, each with whole tiles and with ragged edges
+# 256 x 256, 256 x 128, 128 x 128 in rounds, 128 x 128 alone, 128 x 64 and 64 x 64 tiles, each with whole tiles and with ragged edges; 160 x 128,
+# 192 x 128 and 160 x 64 tiles
 SIZES = [(4096, 4096, 128), (2100, 8200, 64), (1024, 6144, 192), (1000, 6100, 192), (2048, 3072, 128), (2040, 3075, 64), (1280, 2048, 320), (1153, 2047, 64),
-         (512, 1280, 640), (385, 1000, 64), (33, 64, 64), (64, 128, 128), (77, 201, 1088), (257, 513, 64)]
+         (512, 1280, 640), (385, 1000, 64), (33, 64, 64), (64, 128, 128), (77, 201, 1088), (257, 513, 64),
+         (800, 11520, 64), (777, 11460, 192), (576, 21504, 64), (565, 21440, 64), (640, 4096, 128), (565, 4090, 320), (640, 11520, 64), (513, 11516, 128), (193, 4099, 64), (1000, 5100, 64)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

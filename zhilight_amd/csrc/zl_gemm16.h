@@ -160,14 +160,19 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm16(const Gemm16P p, con
 // The tile: the shape whose busiest CU is done first.  `cost` is the measured time of one 64-k slice of one tile (hundredths of a us, cold
 // weights) with the CU as full as the shape's LDS allows, `alone` with one such workgroup per CU; a launch takes ceil(tiles / CUs) of them.  The big
 // tiles win where they come to whole rounds (1024 x 28672: 220 us against 293 with 128 x 128), the deep rings of small tiles where there
-// are fewer tiles than CUs (777 x 2304 x 5760: 36 us with 128 x 64, 77 with 128 x 128 in two slices, 122 with 256 x 256).
+// are fewer tiles than CUs (777 x 2304 x 5760: 36 us with 128 x 64, 77 with 128 x 128 in two slices, 122 with 256 x 256).  160- and 192-row tiles
+// are for heights that the powers of two miss (777 x 11520 x 2304: 48 us with 160 x 128, 70 with 256 x 256; 565 x 21504 x 4096: 97 with 192 x 128,
+// 126 with 256 x 256; 565 x 4096 x 4096: 32 with 160 x 64, 39 with 128 x 128).  The 16-bit tiles of 128 columns that come two to a CU run 4 waves of 64 (80) x 64, a third
+// less LDS traffic per product than 8 of 64 x 32 (4096^3 in 128 x 128: 149 -> 138 us); a workgroup alone on its CU is better off with 8 (2048 x 2048 x
+// 2048 .. 8192 between other kernels: 52 us against 57).
 struct Gemm16Tile { int bm, bn, alone, cost; };
-static const Gemm16Tile kGemm16Tiles[6] = {{256, 256, 185, 172}, {256, 128, 100, 100}, {128, 128, 85, 56}, {128, 128, 61, 62}, {128, 64, 42, 40}, {64, 64, 28, 26}};
+static const Gemm16Tile kGemm16Tiles[9] = {{256, 256, 185, 172}, {256, 128, 100, 100}, {128, 128, 80, 54}, {128, 128, 60, 61}, {128, 64, 42, 40}, {64, 64, 28, 26},
+                                           {160, 128, 78, 62}, {192, 128, 104, 74}, {160, 64, 50, 50}};
 
 static inline int g16_pick(int64_t m, int64_t n) {
     int best = 0;
     int64_t least = INT64_MAX;
-    for (int i = 0; i < 6; ++i) {
+    for (int i = 0; i < 9; ++i) {
         const Gemm16Tile& t = kGemm16Tiles[i];
         const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn), r = (tiles + 255) / 256;
         const int64_t c = r == 1 ? t.alone : r * t.cost;
@@ -197,12 +202,16 @@ int g16_launch_tile(Gemm16P p, const Epi& e, hipStream_t s) {
 
 template <int DT, bool DUAL = false, class Epi>
 int g16_launch(const Gemm16P& p, const Epi& e, hipStream_t s) {
+    constexpr int W128 = DT == G16_I8 ? 4 : 2;                 // (two workgroups per CU; int8's scale-backs are long, more waves share them)
     switch (p.k_part < p.k ? 5 : g16_pick(p.m, p.n)) {         // (a divided k: the caller counts 64 x 64 tiles)
         case 0: return g16_launch_tile<DT, 256, 256, 2, 4, 2, DUAL>(p, e, s);
         case 1: return g16_launch_tile<DT, 256, 128, 4, 2, 3, DUAL>(p, e, s);
-        case 2: return g16_launch_tile<DT, 128, 128, 2, 4, 2, DUAL>(p, e, s);
+        case 2: return g16_launch_tile<DT, 128, 128, 2, W128, 2, DUAL>(p, e, s);
         case 3: return g16_launch_tile<DT, 128, 128, 2, 4, 3, DUAL>(p, e, s);
         case 4: return g16_launch_tile<DT, 128, 64, 4, 2, 4, DUAL>(p, e, s);
+        case 6: return g16_launch_tile<DT, 160, 128, 2, 2, 2, DUAL>(p, e, s);
+        case 7: return g16_launch_tile<DT, 192, 128, 4, 2, 2, DUAL>(p, e, s);
+        case 8: return g16_launch_tile<DT, 160, 64, 2, 2, 3, DUAL>(p, e, s);
         default: return g16_launch_tile<DT, 64, 64, 2, 2, 4, DUAL>(p, e, s);
     }
 }
