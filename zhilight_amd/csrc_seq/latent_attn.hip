@@ -8,10 +8,11 @@
 // identity columns for it (W_uk) or zeros (W_uv) on the host, and every kernel below sees one longer "latent".
 // k_latent_store        RMS norm (plain weight) of the down-projection -> the token's cache row; the rotated key part behind it and the
 //                       queries' rotated parts (in place), turned by the token's position
-// k_latent_absorb       the query folded through W_uk (and the scale), once per token and head
+// k_latent_absorb       the query folded through W_uk (and the scale), once per token and head, 8 tokens to a workgroup
 // k_latent_split        single tokens (and, in 32-bit serving, every token): the keys split over workgroups, fp32 VALU
 // k_latent_decode_mfma  the same split pass for bf16 on the matrix cores
-// k_latent_combine      merges the splits with the sink (it counts once, unscaled, with no value), applies W_uv and the gate
+// k_latent_combine_v    merges the splits with the sink (it counts once, unscaled, with no value), applies W_uv and the gate, 8 tokens to a
+//                       workgroup; k_latent_combine keeps ranks that are no whole 8s and very many splits
 // k_latent_fa           portions of prompts in bf16 on the matrix cores, over keys and values up-projected for the step
 #include "seq_common.h"
 
@@ -56,47 +57,115 @@ struct AttnP {
     const float* q; const float* gate; const void* w_uk; const void* w_uv; const float* sink; const void* cache; void* out;
     int64_t ldq, ldg;
     int q_col0, g_col0, heads, dim, vdim, rank, single_only, vec;
+    int pairs;                                     // W_uk's rows are even and aligned: two columns per load
     float scale;
     int window;                                    // > 0: a token at position p sees the keys p - window < j <= p only
 };
 
-// Split over keys: workgroup = (token, group of 4 heads, split), a wave per head.  A tile of 16 cached rows is staged once in LDS as fp32
-// (row stride rank + 4) and shared by the four heads.  Scores: lane = (key, quarter of the latent columns), two butterflies; weighted sum:
-// a lane owns the latent columns lane, lane + 64, ... (RPL of them, in registers).  Every split leaves (max, denominator, sums) in the
-// workspace; k_latent_combine merges them WITH the sink (m = max(sink, m_i), l = e^(sink - m) + sum l_i e^(m_i - m)), applies W_uv and the
-// gate.  LDS: ct[16][rank + 4] | qk[4][rank]
-// q'_h = scale * W_uk,h^T q_h, once per (token, head): workgroup = 64 latent columns (lanes: coalesced rows of W_uk), the four waves
-// take every fourth query dimension, eight loads in flight each; the partial sums meet in LDS.  qa (n_tok, heads, rank) fp32
+// the workspace: the splits' sums (n_tok, heads, n_splits, rank), the folded queries (n_tok, heads, rank), the splits' (maximum, denominator)
+struct LatWs {
+    float* acc; float2* ml;
+    __device__ __forceinline__ LatWs(float* ws, int n_tok, const AttnP& p, int n_splits, int t, int h, int split) {
+        const size_t at = ((size_t)t * p.heads + h) * n_splits + split;
+        acc = ws + at * p.rank;
+        ml = reinterpret_cast<float2*>(ws + (size_t)n_tok * p.heads * (n_splits + 1) * p.rank) + at;
+    }
+    // (4-byte aligned only when rank is odd)
+    __device__ __forceinline__ void store_ml(float m, float l) const { float* f = reinterpret_cast<float*>(ml); f[0] = m; f[1] = l; }
+};
+
+// two consecutive numbers as they lie in memory: what is converted only after every load is on its way
+template <int DT> struct Raw2;
+template <> struct Raw2<ZL_BF16> {
+    uint32_t u;
+    __device__ __forceinline__ void load(const void* p, size_t i) { u = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(p) + i); }
+    __device__ __forceinline__ void load1(const void* p, size_t i, size_t k) {
+        const uint16_t* h = reinterpret_cast<const uint16_t*>(p);
+        u = h[i] | (uint32_t)h[k] << 16;
+    }
+    __device__ __forceinline__ float2 get() const { return make_float2(__builtin_bit_cast(float, u << 16), __builtin_bit_cast(float, u & 0xffff0000u)); }
+};
+template <> struct Raw2<ZL_F32> {
+    float2 v;
+    __device__ __forceinline__ void load(const void* p, size_t i) { v = *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(p) + i); }
+    __device__ __forceinline__ void load1(const void* p, size_t i, size_t k) { const float* f = reinterpret_cast<const float*>(p); v = make_float2(f[i], f[k]); }
+    __device__ __forceinline__ float2 get() const { return v; }
+};
+
+constexpr int kLatTok = 8;                         // tokens that share a workgroup's weights
+
+// which of the kLatTok tokens from t0 are this kernel's (portions of several tokens go to the prompt kernel); workgroup-uniform
+__device__ __forceinline__ uint32_t lat_live(const AttnP& p, const zls_batch_t& b, int t0) {
+    const int t = t0 + (threadIdx.x & (kLatTok - 1));           // (a lane each: one chain of loads instead of eight)
+    bool live = t < b.n_tok;
+    if (live && p.single_only) {
+        const int sq = b.tok_seq[t];
+        live = b.seq_start[sq + 1] - b.seq_start[sq] <= 1;
+    }
+    return (uint32_t)__ballot(live) & ((1u << kLatTok) - 1);
+}
+
+// q'_h = scale * W_uk,h^T q_h, once per (token, head): workgroup = 64 latent columns (2 per thread) of one head for 8 tokens, its eight half-waves
+// take every eighth query dimension, 16 rows' loads in flight each; the partial sums meet in LDS.  qa (n_tok, heads, rank) fp32.  What bounds it is the
+// latency of W_uk's loads; with a workgroup per token the matrix also came from L2 once per token (8 tokens x 32 heads x 128 x 512: 18 -> 5.8 us)
 template <int DT>
 __global__ __launch_bounds__(256) void k_latent_absorb(const AttnP p, const zls_batch_t b, float* __restrict__ qa) {
-    __shared__ float part[4][64];
-    const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int sq = b.tok_seq[t];
-    if (p.single_only && b.seq_start[sq + 1] - b.seq_start[sq] > 1) return;
-    const float* qh = p.q + (size_t)t * p.ldq + p.q_col0 + (size_t)h * p.dim;
-    const int r = blockIdx.z * 64 + lane;
-    float acc = 0.f;
-    if (r < p.rank) {
-        for (int d0 = wave; d0 < p.dim; d0 += 32) {
-            float w[8];
+    __shared__ __attribute__((aligned(16))) float qs[128][kLatTok];
+    __shared__ float part[8][kLatTok][64];
+    const int t0 = blockIdx.x * kLatTok, h = blockIdx.y, cp = threadIdx.x & 31, grp = threadIdx.x >> 5;
+    const uint32_t live = lat_live(p, b, t0);
+    if (!live) return;
+    const int c = blockIdx.z * 64 + 2 * cp, c0 = min(c, p.rank - 1), c1 = min(c + 1, p.rank - 1);      // (columns past the rank: the last one, never stored)
+    float acc[kLatTok][2];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int d = d0 + 4 * u;
-                w[u] = d < p.dim ? SeqT<DT>::ld(p.w_uk, ((size_t)h * p.dim + d) * p.rank + r) : 0.f;
+    for (int i = 0; i < kLatTok; ++i) acc[i][0] = acc[i][1] = 0.f;
+    for (int d0 = 0; d0 < p.dim; d0 += 128) {
+        Raw2<DT> w[16];
+        if (p.pairs) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) w[u].load(p.w_uk, ((size_t)h * p.dim + min(d0 + grp + 8 * u, p.dim - 1)) * p.rank + (c0 & ~1));
+        } else {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                const size_t row = ((size_t)h * p.dim + min(d0 + grp + 8 * u, p.dim - 1)) * p.rank;
+                w[u].load1(p.w_uk, row + c0, row + c1);
             }
+        }
+        if (d0) __syncthreads();
+        for (int i = threadIdx.x; i < 128 * kLatTok; i += 256) {
+            const int d = i & 127, tk = i >> 7;
+            qs[d][tk] = (live >> tk & 1) && d0 + d < p.dim ? p.q[(size_t)(t0 + tk) * p.ldq + p.q_col0 + (size_t)h * p.dim + d0 + d] : 0.f;
+        }
+        __syncthreads();
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int d = d0 + 4 * u;
-                acc = fmaf(d < p.dim ? qh[d] : 0.f, w[u], acc);
+        for (int u = 0; u < 16; ++u) {
+            const float2 wv = w[u].get();
+#pragma unroll
+            for (int i = 0; i < kLatTok; ++i) {
+                const float qv = qs[grp + 8 * u][i];               // (0 past the last dimension)
+                acc[i][0] = fmaf(qv, wv.x, acc[i][0]);
+                acc[i][1] = fmaf(qv, wv.y, acc[i][1]);
             }
         }
     }
-    part[wave][lane] = acc;
+#pragma unroll
+    for (int i = 0; i < kLatTok; ++i) { part[grp][i][2 * cp] = acc[i][0]; part[grp][i][2 * cp + 1] = acc[i][1]; }
     __syncthreads();
-    if (wave == 0 && r < p.rank)
-        qa[((size_t)t * p.heads + h) * p.rank + r] = (part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane]) * p.scale;
+    for (int i = threadIdx.x; i < kLatTok * 64; i += 256) {
+        const int tk = i >> 6, cc = i & 63, r = blockIdx.z * 64 + cc;
+        if (!(live >> tk & 1) || r >= p.rank) continue;
+        float a = 0.f;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) a += part[g][tk][cc];
+        qa[((size_t)(t0 + tk) * p.heads + h) * p.rank + r] = a * p.scale;
+    }
 }
 
+// Split over keys: workgroup = (token, group of 4 heads, split), a wave per head.  A tile of 16 cached rows is staged once in LDS as fp32
+// (row stride rank + 4) and shared by the four heads.  Scores: lane = (key, quarter of the latent columns), two butterflies; weighted sum:
+// a lane owns the latent columns lane, lane + 64, ... (RPL of them, in registers).  Every split leaves (max, denominator, sums) in the
+// workspace; the combine merges them WITH the sink (m = max(sink, m_i), l = e^(sink - m) + sum l_i e^(m_i - m)), applies W_uv and the
+// gate.  LDS: ct[16][rank + 4] | qk[4][rank]
 template <int DT, int RPL>
 __global__ __launch_bounds__(256) void k_latent_split(const AttnP p, const zls_batch_t b, const float* __restrict__ qa, float* __restrict__ ws,
                                                       int n_splits) {
@@ -210,40 +279,40 @@ __global__ __launch_bounds__(256) void k_latent_split(const AttnP p, const zls_b
         }
     }
     if (!hvalid) return;
-    float* out = ws + (((size_t)t * p.heads + h) * n_splits + split) * (p.rank + 2);
-    if (lane == 0) { out[0] = m; out[1] = l; }
+    const LatWs o(ws, b.n_tok, p, n_splits, t, h, split);
+    if (lane == 0) o.store_ml(m, l);
 #pragma unroll
     for (int i = 0; i < RPL; ++i) {
         const int r = lane + 64 * i;
-        if (r < p.rank) out[2 + r] = acc[i];
+        if (r < p.rank) o.acc[r] = acc[i];
     }
 }
 
 // LDS: acc[rank] | wgt[n_splits]
 template <int DT>
-__global__ __launch_bounds__(256) void k_latent_combine(const AttnP p, const zls_batch_t b, const float* __restrict__ ws, int n_splits) {
+__global__ __launch_bounds__(256) void k_latent_combine(const AttnP p, const zls_batch_t b, float* __restrict__ ws, int n_splits) {
     extern __shared__ float lds[];
     __shared__ float red[16];
     float* wgt = lds + p.rank;
     const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int sq = b.tok_seq[t];
     if (p.single_only && b.seq_start[sq + 1] - b.seq_start[sq] > 1) return;
-    const float* part = ws + ((size_t)t * p.heads + h) * n_splits * (p.rank + 2);
+    const LatWs part(ws, b.n_tok, p, n_splits, t, h, 0);
     float mloc = p.sink ? p.sink[h] : -INFINITY;                       // threads along the splits: loads in parallel
-    for (int s2 = threadIdx.x; s2 < n_splits; s2 += 256) mloc = fmaxf(mloc, part[(size_t)s2 * (p.rank + 2)]);
+    for (int s2 = threadIdx.x; s2 < n_splits; s2 += 256) mloc = fmaxf(mloc, reinterpret_cast<const float*>(part.ml)[2 * s2]);
     const float m = zl_block_max(mloc, red);
     float lloc = 0.f;
     for (int s2 = threadIdx.x; s2 < n_splits; s2 += 256) {
-        const float ms = part[(size_t)s2 * (p.rank + 2)];
+        const float ms = reinterpret_cast<const float*>(part.ml)[2 * s2];
         const float w = ms == -INFINITY ? 0.f : expf(ms - m);
         wgt[s2] = w;
-        lloc = fmaf(part[(size_t)s2 * (p.rank + 2) + 1], w, lloc);
+        lloc = fmaf(reinterpret_cast<const float*>(part.ml)[2 * s2 + 1], w, lloc);
     }
     const float l = zl_block_sum(lloc, red) + (p.sink ? expf(p.sink[h] - m) : 0.f);      // (its barriers also publish wgt)
     for (int r = threadIdx.x; r < p.rank; r += 256) {
         float a = 0.f;
 #pragma unroll 8
-        for (int s2 = 0; s2 < n_splits; ++s2) a = fmaf(part[(size_t)s2 * (p.rank + 2) + 2 + r], wgt[s2], a);
+        for (int s2 = 0; s2 < n_splits; ++s2) a = fmaf(part.acc[(size_t)s2 * p.rank + r], wgt[s2], a);
         lds[r] = a;
     }
     __syncthreads();
@@ -265,6 +334,134 @@ __global__ __launch_bounds__(256) void k_latent_combine(const AttnP p, const zls
             if (lane == 0 && d0 + u < p.vdim) SeqT<DT>::st(p.out, ((size_t)t * p.heads + h) * p.vdim + d0 + u, v * inv);
         }
     }
+}
+
+// the same for ranks of whole 8s: workgroup = 16 outputs of one head for 8 tokens, whose rows of W_uv are on the way while the splits are merged
+// (a wave per token's weights, then 16-byte pieces of the sums); a wave = 4 outputs, a lane = 8 latent columns of each row for all the tokens, and
+// the 32 sums of a wave are exchanged down to one per pair of lanes.  LDS: lat[8][rank] | wgt[8][n_splits] | inv[8]
+// (8 tokens x 32 heads x 128 x 512: 31 -> 9.3 us: W_uv came from L2 once per token, and every wave sum took six exchanges)
+template <int DT> struct Raw8;
+template <> struct Raw8<ZL_BF16> {
+    uint4 r;
+    __device__ __forceinline__ void load(const void* p, size_t i) { r = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p) + i); }
+    __device__ __forceinline__ void clear() { r = make_uint4(0, 0, 0, 0); }
+    __device__ __forceinline__ void get(float* v) const {
+        const uint32_t u[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { v[2 * e] = __builtin_bit_cast(float, u[e] << 16); v[2 * e + 1] = __builtin_bit_cast(float, u[e] & 0xffff0000u); }
+    }
+};
+template <> struct Raw8<ZL_F32> {
+    float4 a, c;
+    __device__ __forceinline__ void load(const void* p, size_t i) { const float* f = reinterpret_cast<const float*>(p) + i; a = seq_ld4(f); c = seq_ld4(f + 4); }
+    __device__ __forceinline__ void clear() { a = c = make_float4(0.f, 0.f, 0.f, 0.f); }
+    __device__ __forceinline__ void get(float* v) const { v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = c.x; v[5] = c.y; v[6] = c.z; v[7] = c.w; }
+};
+
+// lanes whose numbers differ in bit 2 N swap halves of v[0 .. 2 N): half as many sums per lane, each over twice as many lanes
+template <int N>
+__device__ __forceinline__ void lat_fold(float* v, int lane) {
+    const bool up = lane & (2 * N);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float keep = up ? v[i + N] : v[i], send = up ? v[i] : v[i + N];
+        v[i] = keep + __shfl_xor(send, 2 * N, 64);
+    }
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void k_latent_combine_v(const AttnP p, const zls_batch_t b, float* __restrict__ ws, int n_splits) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    float* lat = lds;
+    float* wgt = lds + kLatTok * p.rank;
+    float* inv = wgt + kLatTok * n_splits;
+    const int t0 = blockIdx.x * kLatTok, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t live = lat_live(p, b, t0);
+    if (!live) return;
+    const int d0 = blockIdx.z * 16 + wave * 4;
+    Raw8<DT> w[4];
+    auto rows = [&](int c) {                                               // 8 columns from c of the wave's 4 rows of W_uv
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (d0 + u < p.vdim && c < p.rank) w[u].load(p.w_uv, ((size_t)h * p.vdim + d0 + u) * p.rank + c);
+            else w[u].clear();
+        }
+    };
+    rows(8 * lane);
+    const float sink = p.sink ? p.sink[h] : -INFINITY;
+    for (int tk = wave; tk < kLatTok; tk += 4) {
+        if (!(live >> tk & 1)) continue;
+        const LatWs part(ws, b.n_tok, p, n_splits, t0 + tk, h, 0);
+        float m = sink;
+        for (int s = lane; s < n_splits; s += 64) m = fmaxf(m, part.ml[s].x);
+        m = zl_wave_max(m);
+        float l = 0.f;
+        for (int s = lane; s < n_splits; s += 64) {
+            const float2 v = part.ml[s];
+            const float e = v.x == -INFINITY ? 0.f : expf(v.x - m);
+            wgt[tk * n_splits + s] = e;
+            l = fmaf(v.y, e, l);
+        }
+        l = zl_wave_sum(l) + (p.sink ? expf(sink - m) : 0.f);
+        if (lane == 0) inv[tk] = (p.gate ? seq_sigmoid(p.gate[(size_t)(t0 + tk) * p.ldg + p.g_col0 + h]) : 1.0f) / l;
+    }
+    __syncthreads();
+    const int quads = p.rank >> 2;
+    const float* acc = LatWs(ws, b.n_tok, p, n_splits, t0, h, 0).acc;
+    const size_t tok = (size_t)p.heads * n_splits * p.rank;                // (the next token's sums of this head)
+    for (int i0 = threadIdx.x; i0 < kLatTok * quads; i0 += 1024) {         // 4 pieces of 4 splits in flight per thread
+        float4 a[4];
+        int tk[4], at[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = min(i0 + 256 * u, kLatTok * quads - 1);          // (past the end: the last piece once more)
+            tk[u] = i / quads; at[u] = (i - tk[u] * quads) * 4;
+            a[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        for (int s0 = 0; s0 < n_splits; s0 += 4) {
+            float4 x[4][4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)                                // (tokens of other kernels: the room is there, the numbers are not used)
+                    x[u][e] = seq_ld4(acc + min(tk[u], b.n_tok - 1 - t0) * tok + (size_t)min(s0 + e, n_splits - 1) * p.rank + at[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (s0 + e >= n_splits || !(live >> tk[u] & 1)) continue;
+                    const float f = wgt[tk[u] * n_splits + s0 + e];
+                    a[u] = make_float4(fmaf(x[u][e].x, f, a[u].x), fmaf(x[u][e].y, f, a[u].y), fmaf(x[u][e].z, f, a[u].z), fmaf(x[u][e].w, f, a[u].w));
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) *reinterpret_cast<float4*>(lat + (size_t)tk[u] * p.rank + at[u]) = a[u];
+    }
+    __syncthreads();
+    float v[4 * kLatTok];                                                  // [output][token]
+#pragma unroll
+    for (int i = 0; i < 4 * kLatTok; ++i) v[i] = 0.f;
+    for (int c = 8 * lane; c < p.rank; c += 512) {
+        if (c >= 512) rows(c);
+        float wf[4][8];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) w[u].get(wf[u]);
+#pragma unroll
+        for (int tk = 0; tk < kLatTok; ++tk) {
+            if (!(live >> tk & 1)) continue;
+            const float4 x = seq_ld4(lat + (size_t)tk * p.rank + c), y = seq_ld4(lat + (size_t)tk * p.rank + c + 4);
+            const float xv[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[u * kLatTok + tk] = fmaf(wf[u][e], xv[e], v[u * kLatTok + tk]);
+        }
+    }
+    // lanes 2 i and 2 i + 1 end up with the whole sum of v[i]
+    lat_fold<16>(v, lane); lat_fold<8>(v, lane); lat_fold<4>(v, lane); lat_fold<2>(v, lane); lat_fold<1>(v, lane);
+    const float sum = v[0] + __shfl_xor(v[0], 1, 64);
+    const int tk = (lane >> 1) & 7, d = d0 + (lane >> 4);
+    if (!(lane & 1) && (live >> tk & 1) && d < p.vdim) SeqT<DT>::st(p.out, ((size_t)(t0 + tk) * p.heads + h) * p.vdim + d, sum * inv[tk]);
 }
 
 // ---- prompt portions on the matrix cores (bf16 serving) -----------------------------------------------------------------------------
@@ -464,18 +661,21 @@ __global__ __launch_bounds__(256) void k_latent_fa(const FaP p, const zls_batch_
 }
 
 // ---- single tokens in bf16 on the matrix cores --------------------------------------------------------------------------------------
-// One wave = one token x 16 heads x one split of the keys.  Per 32 keys: the latent rows go from the pages straight into A operands
-// (lane = key, 8 consecutive latent columns per 16-byte load), S^T (16 keys x 16 heads) = C . Q'^T with the folded queries as B operands
-// held in registers; softmax per lane (= per head) as in the prompt kernel; the rows are then parked in LDS and read back column-wise for
-// O^T (latent x 16 heads) += C^T . P^T (the contraction runs over the 32 keys in the order the scores lie in the lanes; two bf16 halves
-// per weight).  Leaves (max, denominator, sums) per split in the workspace of k_latent_split's format: k_latent_combine finishes both.
-template <int RT>                                                                  // rank <= 32 RT
-__global__ __launch_bounds__(64) void k_latent_decode_mfma(const AttnP p, const zls_batch_t b, const float* __restrict__ qa,
-                                                           float* __restrict__ ws, int n_splits) {
-    constexpr int CR = RT * 32 + 8;
-    __shared__ __attribute__((aligned(16))) uint16_t ct[32 * CR];
-    const int t = blockIdx.x, split = blockIdx.z, lane = threadIdx.x, nrow = lane & 15, kq = lane >> 4;
-    const int head = blockIdx.y * 16 + nrow;
+// Workgroup = one token x 16 heads x one split of the keys; its NW waves divide the latent's columns, RW blocks of 32 each.  Per 32 keys a wave's
+// columns go from the pages straight into A operands (lane = key, 8 consecutive columns per 16-byte load, the next block's on the way), S^T
+// (16 keys x 16 heads) += C . Q'^T with the folded queries as B operands held in registers; the waves' partial scores meet in LDS, every wave
+// does the softmax per lane (= per head) as in the prompt kernel; the columns are parked in LDS by the wave that owns them and read back
+// column-wise for O^T (latent x 16 heads) += C^T . P^T (the contraction runs over the 32 keys in the order the scores lie in the lanes; two bf16
+// halves per weight).  What bounds it is this chain per block: one wave did all columns before, 32 waves in all for 8 tokens of 130 keys (35 -> 11 us).
+// Leaves (max, denominator, sums) per split in the workspace as k_latent_split does.
+template <int RW, int NW>                                                          // rank <= 32 RW NW
+__global__ __launch_bounds__(64 * NW) void k_latent_decode_mfma(const AttnP p, const zls_batch_t b, const float* __restrict__ qa,
+                                                                float* __restrict__ ws, int n_splits) {
+    constexpr int CR = RW * 32 + 8;
+    __shared__ __attribute__((aligned(16))) uint16_t ct_all[NW][32 * CR];
+    __shared__ __attribute__((aligned(16))) float4 part[2][NW][2][64];
+    const int t = blockIdx.x, split = blockIdx.z, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nrow = lane & 15, kq = lane >> 4;
+    const int head = blockIdx.y * 16 + nrow, r0 = wave * RW * 32;
     const bool hvalid = head < p.heads;
     const int sq = b.tok_seq[t];
     if (p.single_only && b.seq_start[sq + 1] - b.seq_start[sq] > 1) return;
@@ -486,48 +686,69 @@ __global__ __launch_bounds__(64) void k_latent_decode_mfma(const AttnP p, const 
     const int k0 = key_lo + split * chunk, k1 = min(pos + 1, k0 + chunk);
     const int32_t* pages = b.page_table + (size_t)sq * b.max_pages;
     const uint16_t* cache = reinterpret_cast<const uint16_t*>(p.cache);
+    uint16_t* ct = ct_all[wave];
 
-    uint4 qf[RT];
-    {
-        const float* qr = qa + ((size_t)t * p.heads + (hvalid ? head : 0)) * p.rank;
-#pragma unroll
-        for (int kk = 0; kk < RT; ++kk) {
-            uint32_t w[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int r = 32 * kk + 8 * kq + 2 * i;
-                const float a = (hvalid && r < p.rank) ? qr[r] : 0.f, c = (hvalid && r + 1 < p.rank) ? qr[r + 1] : 0.f;
-                w[i] = ZT<ZL_BF16>::from_f32(a) | (uint32_t)ZT<ZL_BF16>::from_f32(c) << 16;
-            }
-            qf[kk] = make_uint4(w[0], w[1], w[2], w[3]);
-        }
-    }
-    fa_f4 o[2 * RT];
-#pragma unroll
-    for (int rt = 0; rt < 2 * RT; ++rt) o[rt] = (fa_f4){0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
-
-    for (int j0 = k0; j0 < k1; j0 += 32) {
-        uint4 cr[2][RT];
+    uint4 cr[2][RW];
+    auto fetch = [&](int j0) {
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             const int j = j0 + 16 * c + nrow;
             const bool valid = j < k1;
             const size_t base = valid ? ((size_t)pages[j / b.page_size] * b.page_size + j % b.page_size) * p.rank : 0;
 #pragma unroll
-            for (int kk = 0; kk < RT; ++kk) {
-                const int r = 32 * kk + 8 * kq;
+            for (int kk = 0; kk < RW; ++kk) {
+                const int r = r0 + 32 * kk + 8 * kq;
                 cr[c][kk] = (valid && r < p.rank) ? *reinterpret_cast<const uint4*>(cache + base + r) : make_uint4(0, 0, 0, 0);
             }
         }
+    };
+    if (k0 < k1) fetch(k0);
+    uint4 qf[RW];
+    {
+        const float* qr = qa + ((size_t)t * p.heads + (hvalid ? head : 0)) * p.rank;
+#pragma unroll
+        for (int kk = 0; kk < RW; ++kk) {
+            const int r = r0 + 32 * kk + 8 * kq;
+            const bool in = hvalid && r < p.rank;                                  // (rank comes in whole 8s)
+            const float4 a = in ? seq_ld4(qr + r) : make_float4(0.f, 0.f, 0.f, 0.f), c = in ? seq_ld4(qr + r + 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+            qf[kk] = make_uint4(ZT<ZL_BF16>::from_f32(a.x) | (uint32_t)ZT<ZL_BF16>::from_f32(a.y) << 16, ZT<ZL_BF16>::from_f32(a.z) | (uint32_t)ZT<ZL_BF16>::from_f32(a.w) << 16,
+                                ZT<ZL_BF16>::from_f32(c.x) | (uint32_t)ZT<ZL_BF16>::from_f32(c.y) << 16, ZT<ZL_BF16>::from_f32(c.z) | (uint32_t)ZT<ZL_BF16>::from_f32(c.w) << 16);
+        }
+    }
+    fa_f4 o[2 * RW];
+#pragma unroll
+    for (int rt = 0; rt < 2 * RW; ++rt) o[rt] = (fa_f4){0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    int turn = 0;
+    for (int j0 = k0; j0 < k1; j0 += 32, turn ^= 1) {
         fa_f4 sc[2];
-        float mx = -INFINITY;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             sc[c] = (fa_f4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int kk = 0; kk < RT; ++kk)
+            for (int kk = 0; kk < RW; ++kk)
                 sc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(fa_b8, cr[c][kk]), __builtin_bit_cast(fa_b8, qf[kk]), sc[c], 0, 0, 0);
+            if (NW > 1) part[turn][wave][c][lane] = make_float4(sc[c][0], sc[c][1], sc[c][2], sc[c][3]);
+        }
+        // (the wave's own reads of the last block's columns came before these writes, LDS keeps a wave's order)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int kk = 0; kk < RW; ++kk) *reinterpret_cast<uint4*>(ct + (16 * c + nrow) * CR + 32 * kk + 8 * kq) = cr[c][kk];
+        if (j0 + 32 < k1) fetch(j0 + 32);
+        __syncthreads();                                                           // (one per block: the partial scores alternate between two places)
+        float mx = -INFINITY;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            if (NW > 1) {
+                float4 a = part[turn][0][c][lane];
+#pragma unroll
+                for (int w = 1; w < NW; ++w) {
+                    const float4 v = part[turn][w][c][lane];
+                    a = make_float4(a.x + v.x, a.y + v.y, a.z + v.z, a.w + v.w);
+                }
+                sc[c] = (fa_f4){a.x, a.y, a.z, a.w};
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float v = (j0 + 16 * c + 4 * kq + r < k1) ? sc[c][r] : -INFINITY;        // (the folded query carries the scale)
@@ -562,15 +783,9 @@ __global__ __launch_bounds__(64) void k_latent_decode_mfma(const AttnP p, const 
         m = mnew;
         const fa_b8 ph = __builtin_bit_cast(fa_b8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
         const fa_b8 pl = __builtin_bit_cast(fa_b8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
-        __syncthreads();                                                           // the previous block's column reads are done
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-            for (int kk = 0; kk < RT; ++kk) *reinterpret_cast<uint4*>(ct + (16 * c + nrow) * CR + 32 * kk + 8 * kq) = cr[c][kk];
-        __syncthreads();
-#pragma unroll
-        for (int rt = 0; rt < 2 * RT; ++rt) {
-            // slot s of lane group kq <-> key 16 (s / 4) + 4 kq + s % 4 of the block; this lane's column of the latent: 16 rt + nrow
+        for (int rt = 0; rt < 2 * RW; ++rt) {
+            // slot s of lane group kq <-> key 16 (s / 4) + 4 kq + s % 4 of the block; this lane's column of the wave's part: 16 rt + nrow
             uint32_t w[4];
 #pragma unroll
             for (int s2 = 0; s2 < 4; ++s2) {
@@ -584,15 +799,13 @@ __global__ __launch_bounds__(64) void k_latent_decode_mfma(const AttnP p, const 
         }
     }
     if (!hvalid) return;
-    float* out = ws + (((size_t)t * p.heads + head) * n_splits + split) * (p.rank + 2);
-    if (kq == 0) { out[0] = m; out[1] = l; }
+    const LatWs out(ws, b.n_tok, p, n_splits, t, head, split);
+    if (wave == 0 && kq == 0) *out.ml = make_float2(m, l);
 #pragma unroll
-    for (int rt = 0; rt < 2 * RT; ++rt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 16 * rt + 4 * kq + i;
-            if (r < p.rank) out[2 + r] = o[rt][i];
-        }
+    for (int rt = 0; rt < 2 * RW; ++rt) {
+        const int r = r0 + 16 * rt + 4 * kq;
+        if (r < p.rank) *reinterpret_cast<float4*>(out.acc + r) = make_float4(o[rt][0], o[rt][1], o[rt][2], o[rt][3]);
+    }
 }
 
 }  // namespace
@@ -617,7 +830,7 @@ extern "C" int zls_latent_store(const float* proj, int64_t ld, int64_t col0, con
 
 extern "C" int64_t zls_latent_attention_workspace_bytes(int64_t n_tok, int64_t heads, int64_t rank, int64_t n_splits) {
     if (n_tok <= 0 || heads <= 0 || rank <= 0 || n_splits <= 0) return ZL_EINVAL;
-    return (n_tok * heads * n_splits * (rank + 2) + n_tok * heads * rank) * (int64_t)sizeof(float);    /* partials | folded queries */
+    return (n_tok * heads * n_splits * (rank + 2) + n_tok * heads * rank) * (int64_t)sizeof(float);    /* sums, (maximum, denominator) | folded queries */
 }
 
 extern "C" int zls_latent_attention(const float* q, int64_t ldq, int64_t q_col0, const float* gate, int64_t ldg, int64_t g_col0, const void* w_uk,
@@ -640,28 +853,34 @@ extern "C" int zls_latent_attention(const float* q, int64_t ldq, int64_t q_col0,
     const dim3 grid(b->n_tok, (unsigned)((heads + 3) / 4), (unsigned)n_splits);
     hipStream_t hs = (hipStream_t)s;
     float* ws = (float*)workspace;
-    float* qa = ws + (size_t)b->n_tok * heads * n_splits * (rank + 2);
+    float* qa = ws + (size_t)b->n_tok * heads * n_splits * rank;
     const int ns = (int)n_splits;
     // bf16 with aligned rows of at most 640 latent columns (512 + a rotated part): the split pass on the matrix cores (absorb and combine
     // are shared)
-    const bool mfma = dtype == ZL_BF16 && p.vec && rank <= 640 && !no_mfma;
+    const bool ws16 = ((uintptr_t)workspace & 15) == 0;
+    const bool mfma = dtype == ZL_BF16 && p.vec && ws16 && rank <= 640 && !no_mfma;
+    p.pairs = rank % 2 == 0 && ((uintptr_t)w_uk & 7) == 0;
+    const unsigned tgrid = (unsigned)((b->n_tok + kLatTok - 1) / kLatTok);
+    const size_t lds_v = (size_t)(kLatTok * (rank + n_splits) + kLatTok) * sizeof(float);
+    const bool rows8 = rank % 8 == 0 && ws16 && ((uintptr_t)w_uv & 15) == 0 && lds_v <= 64 * 1024;
     const dim3 mgrid(b->n_tok, (unsigned)((heads + 15) / 16), (unsigned)n_splits);
-#define MSPLIT(RT) hipLaunchKernelGGL((k_latent_decode_mfma<RT>), mgrid, dim3(64), 0, hs, p, *b, qa, ws, ns)
+#define MSPLIT(RW, NW) hipLaunchKernelGGL((k_latent_decode_mfma<RW, NW>), mgrid, dim3(64 * NW), 0, hs, p, *b, qa, ws, ns)
 #define SPLIT(DT, RPL) hipLaunchKernelGGL((k_latent_split<DT, RPL>), grid, dim3(256), lds, hs, p, *b, qa, ws, ns)
 #define CALL(DT)                                  \
-    hipLaunchKernelGGL((k_latent_absorb<DT>), dim3(b->n_tok, (unsigned)heads, (unsigned)((rank + 63) / 64)), dim3(256), 0, hs, p, *b, qa); \
+    hipLaunchKernelGGL((k_latent_absorb<DT>), dim3(tgrid, (unsigned)heads, (unsigned)((rank + 63) / 64)), dim3(256), 0, hs, p, *b, qa); \
     if (mfma) {                                   \
-        if (rank <= 64) MSPLIT(2);                \
-        else if (rank <= 128) MSPLIT(4);          \
-        else if (rank <= 256) MSPLIT(8);          \
-        else if (rank <= 512) MSPLIT(16);         \
-        else MSPLIT(20);                          \
+        if (rank <= 64) MSPLIT(1, 2);             \
+        else if (rank <= 128) MSPLIT(1, 4);       \
+        else if (rank <= 256) MSPLIT(2, 4);       \
+        else if (rank <= 512) MSPLIT(4, 4);       \
+        else MSPLIT(5, 4);                        \
     } else if (rank <= 64) SPLIT(DT, 1);          \
     else if (rank <= 128) SPLIT(DT, 2);           \
     else if (rank <= 256) SPLIT(DT, 4);           \
     else if (rank <= 512) SPLIT(DT, 8);           \
     else SPLIT(DT, 16);                           \
-    hipLaunchKernelGGL((k_latent_combine<DT>), dim3(b->n_tok, (unsigned)heads, (unsigned)((vdim + 31) / 32 > 4 ? 4 : (vdim + 31) / 32)), dim3(256), (size_t)(rank + n_splits) * sizeof(float), hs, p, *b, ws, ns);
+    if (rows8) hipLaunchKernelGGL((k_latent_combine_v<DT>), dim3(tgrid, (unsigned)heads, (unsigned)((vdim + 15) / 16)), dim3(256), lds_v, hs, p, *b, ws, ns); \
+    else hipLaunchKernelGGL((k_latent_combine<DT>), dim3(b->n_tok, (unsigned)heads, (unsigned)((vdim + 31) / 32 > 4 ? 4 : (vdim + 31) / 32)), dim3(256), (size_t)(rank + n_splits) * sizeof(float), hs, p, *b, ws, ns);
     ZLS_DISPATCH(dtype, CALL)
 #undef CALL
 #undef SPLIT

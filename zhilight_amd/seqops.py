@@ -365,11 +365,15 @@ def latent_attention(q, q_col0, gate, g_col0, w_uk, w_uv, sink, cache, batch, sc
         raise ZLError("latent_attention: one sink per head")
     if out is None:
         out = torch.empty((batch.n_tok, heads * vdim), dtype=cache.dtype, device=cache.device)
-    # enough workgroups to fill the chip (256 CUs, a few per CU), at least 64 keys per split
-    groups = batch.n_tok * ((heads + 3) // 4)
+    # enough workgroups to fill the chip: in bf16 one of 4 waves per CU and 16 heads, at least 32 keys (a block) each -- the combine reads every
+    # split's sums; else a few per CU and 4 heads, at least 64 keys per split
     if n_splits is None:
         span = min(batch.max_ctx, window) if window > 0 else batch.max_ctx
-        n_splits = max(1, min((span + 63) // 64, (1024 + groups - 1) // groups))
+        if mfma and cache.dtype == torch.bfloat16 and rank % 8 == 0 and rank <= 640:
+            groups, keys, fill = batch.n_tok * ((heads + 15) // 16), 32, 256
+        else:
+            groups, keys, fill = batch.n_tok * ((heads + 3) // 4), 64, 1024
+        n_splits = max(1, min((span + keys - 1) // keys, (fill + groups - 1) // groups))
     ws = torch.empty(int(lib().zls_latent_attention_workspace_bytes(_i(batch.n_tok), _i(heads), _i(rank), _i(n_splits))) // 4,
                      dtype=torch.float32, device=cache.device)
     check(lib().zls_latent_attention(_p(q), _i(q.shape[1]), _i(q_col0), _p(gate), _i(0 if gate is None else gate.shape[1]), _i(g_col0), _p(w_uk),
