@@ -14,6 +14,7 @@
 // k_latent_combine_v    merges the splits with the sink (it counts once, unscaled, with no value), applies W_uv and the gate, 8 tokens to a
 //                       workgroup; k_latent_combine keeps ranks that are no whole 8s and very many splits
 // k_latent_fa           portions of prompts in bf16 on the matrix cores, over keys and values up-projected for the step
+#include <type_traits>
 #include "seq_common.h"
 
 namespace {
@@ -489,64 +490,63 @@ __device__ __forceinline__ void fa_split(float pv, uint16_t& hb, uint16_t& lb) {
 struct FaP {
     const float* q; const float* gate; const uint16_t* k; const uint16_t* vt; const float* sink; const int32_t* ctx_start; uint16_t* out;
     int64_t ldq, ldg, ldk, ldv;
-    int q_col0, g_col0, heads, dim, vdim, tiles_per_seq, vec_k;
+    int q_col0, g_col0, heads, dim, vdim, tiles_per_seq;
     float scale;
     int window; const int32_t* ctx_pos0;           // window > 0: keys p - window < j <= p; ctx_pos0 (nullable: 0): the position of a sequence's
 };                                                 // first up-projected row (a windowed step does not bring its whole context)
 
-template <int DK, int DV>
-__global__ __launch_bounds__(256) void k_latent_fa(const FaP p, const zls_batch_t b) {
-    constexpr int KR = DK * 32 + 8, VR = 64 + 8;
-    __shared__ __attribute__((aligned(16))) uint16_t Ks[64 * KR];
-    __shared__ __attribute__((aligned(16))) uint16_t Vs[DV * 16 * VR];
-    // (the last query tiles see the most keys: they are dispatched first, so the launch does not end on its longest workgroups)
-    const int sq = blockIdx.x % b.n_seq, tile = p.tiles_per_seq - 1 - blockIdx.x / b.n_seq, h = blockIdx.y;
+// NG groups of four waves take a workgroup's key tiles in turn, each with tiles of its own in LDS, and meet at the end: with as many query tiles as a
+// prompt of a few thousand tokens has, the chip holds two workgroups per CU, and a tile's chain of LDS writes, barriers, products and exponentials
+// is what the time goes into (2048 tokens x 16 heads of 128: 123 -> 67 us; masks only where a tile has keys that some query must not see).
+// VEC: heads in whole 8s, rows aligned (others read K and the queries number by number).
+template <int DK, int DV, int NG, bool VEC>
+__global__ __launch_bounds__(256 * NG, NG == 2 && DK <= 4 ? 4 : 1) void k_latent_fa(const FaP p, const zls_batch_t b) {
+    constexpr int KR = DK * 32 + 8, VR = 64 + 8, kGroup = 64 * KR + DV * 16 * VR;
+    static_assert(NG == 1 || 4 * 64 * (DV * 4 + 2) * 4 <= NG * kGroup * 2, "the second group's sums fit");
+    __shared__ __attribute__((aligned(16))) uint16_t smem[NG * kGroup];
+    // The last query tiles see the most keys: they are dispatched first, so the launch does not end on its longest workgroups.  A launch that the
+    // chip holds at once, two workgroups to a CU, is done when its busiest CU is: the second half goes the other way round, the shortest
+    // beside the longest.  (Heads vary fastest: with 8 or 16 of them a head's keys and values stay in one XCD's cache.)
+    const int total = gridDim.x, id = total <= 512 && blockIdx.x >= 256 ? 256 + total - 1 - (int)blockIdx.x : blockIdx.x, per = b.n_seq * p.heads;
+    const int tile = p.tiles_per_seq - 1 - id / per, sq = id % per / p.heads, h = id % p.heads;
     const int first = b.seq_start[sq], count = b.seq_start[sq + 1] - first;
     const int cs = p.ctx_start[sq];
     if (cs < 0 || tile * 64 >= count) return;
     // positions below are counted from the sequence's first up-projected row (position c0): a key's index there is its row in K / V^T
     const int c0 = p.ctx_pos0 ? p.ctx_pos0[sq] : 0;
     const int pos0 = b.seq_pos0[sq] - c0;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nrow = lane & 15, kq = lane >> 4;
+    const int tid = threadIdx.x & 255, lane = tid & 63, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nrow = lane & 15, kq = lane >> 4;
+    uint16_t* Ks = smem + grp * kGroup;
+    uint16_t* Vs = Ks + 64 * KR;
     const int qi = tile * 64 + wave * 16 + nrow;
     const bool qvalid = qi < count;
     const int qpos = pos0 + qi;
     const int j_first = p.window > 0 ? max(0, pos0 + tile * 64 - p.window + 1) & ~63 : 0;     // the tile of the oldest key the first query sees
+    const int wave_first = pos0 + tile * 64 + wave * 16;                           // the wave's first query
     const int wave_last = pos0 + min(count, tile * 64 + wave * 16 + 16) - 1;       // the last key any query of this wave sees
     const int block_last = pos0 + min(count, tile * 64 + 64) - 1;
-
-    uint4 qf[DK];
-    {
-        const float* qr = p.q + (size_t)(first + (qvalid ? qi : 0)) * p.ldq + p.q_col0 + (size_t)h * p.dim;
-#pragma unroll
-        for (int kk = 0; kk < DK; ++kk) {
-            uint32_t w[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int d = 32 * kk + 8 * kq + 2 * i;
-                const float a = (qvalid && d < p.dim) ? qr[d] : 0.f, c = (qvalid && d + 1 < p.dim) ? qr[d + 1] : 0.f;
-                w[i] = ZT<ZL_BF16>::from_f32(a) | (uint32_t)ZT<ZL_BF16>::from_f32(c) << 16;
-            }
-            qf[kk] = make_uint4(w[0], w[1], w[2], w[3]);
-        }
-    }
-    fa_f4 o[DV];
-#pragma unroll
-    for (int dt = 0; dt < DV; ++dt) o[dt] = (fa_f4){0.f, 0.f, 0.f, 0.f};
-    float m = p.sink ? p.sink[h] : -INFINITY, l = p.sink ? 1.0f : 0.0f;
 
     // K and V^T tiles: the NEXT tile's 16-byte loads are issued into registers before the current tile's MFMAs and written to LDS after them
     constexpr int KU = DK, VU = (DV + 1) / 2;                                      // 16-byte units per thread: 64 DK 4 / 256 and DV 16 8 / 256
     uint4 kreg[KU], vreg[VU];
+    constexpr bool kRows = 256 % (DK * 4) == 0;                                    // a thread's units of K lie in one column
+    using offs_t = typename std::conditional<VEC, uint32_t, size_t>::type;          // (VEC: strides below 2^24)
+    const offs_t k_off = (offs_t)(tid / (DK * 4)) * (offs_t)p.ldk + (tid % (DK * 4)) * 8, v_off = (offs_t)(tid >> 3) * (offs_t)p.ldv + (tid & 7) * 8;
     auto fetch_tiles = [&](int j0) {
+        const uint16_t* kb = p.k + (size_t)(cs + j0) * p.ldk + (size_t)h * p.dim;
+        const uint16_t* vb = p.vt + (size_t)h * p.vdim * p.ldv + cs + j0;
 #pragma unroll
         for (int u = 0; u < KU; ++u) {
             const int idx = tid + 256 * u;
             const int key = idx / (DK * 4), d = (idx % (DK * 4)) * 8;
-            const uint16_t* src = p.k + (size_t)(cs + j0 + key) * p.ldk + (size_t)h * p.dim + d;
             uint4 v = make_uint4(0, 0, 0, 0);
-            if (d + 8 <= p.dim && p.vec_k) v = *reinterpret_cast<const uint4*>(src);
-            else if (d < p.dim) {
+            if constexpr (VEC && kRows) {
+                if (d < p.dim) v = *reinterpret_cast<const uint4*>(kb + (size_t)(u * (256 / (DK * 4))) * p.ldk + k_off);
+            } else if constexpr (VEC) {
+                if (d < p.dim) v = *reinterpret_cast<const uint4*>(kb + (size_t)key * p.ldk + d);
+            } else if (d < p.dim) {
+                const uint16_t* src = kb + (size_t)key * p.ldk + d;
                 uint16_t e[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) e[i] = d + i < p.dim ? src[i] : (uint16_t)0;
@@ -557,56 +557,93 @@ __global__ __launch_bounds__(256) void k_latent_fa(const FaP p, const zls_batch_
 #pragma unroll
         for (int u = 0; u < VU; ++u) {
             const int idx = tid + 256 * u;
-            const int d = idx >> 3, c8 = (idx & 7) * 8;
             uint4 v = make_uint4(0, 0, 0, 0);
-            if (idx < DV * 16 * 8 && d < p.vdim) v = *reinterpret_cast<const uint4*>(p.vt + ((size_t)h * p.vdim + d) * p.ldv + cs + j0 + c8);
+            if ((DV % 2 == 0 || idx < DV * 16 * 8) && (idx >> 3) < p.vdim) v = *reinterpret_cast<const uint4*>(vb + (size_t)(u * 32) * p.ldv + v_off);
             vreg[u] = v;
         }
     };
+    uint16_t* const k_to = Ks + (tid / (DK * 4)) * KR + (tid % (DK * 4)) * 8;
+    uint16_t* const v_to = Vs + (tid >> 3) * VR + (tid & 7) * 8;
     auto publish_tiles = [&]() {
 #pragma unroll
         for (int u = 0; u < KU; ++u) {
             const int idx = tid + 256 * u;
-            *reinterpret_cast<uint4*>(Ks + (idx / (DK * 4)) * KR + (idx % (DK * 4)) * 8) = kreg[u];
+            *reinterpret_cast<uint4*>(kRows ? k_to + u * (256 / (DK * 4)) * KR : Ks + (idx / (DK * 4)) * KR + (idx % (DK * 4)) * 8) = kreg[u];
         }
 #pragma unroll
-        for (int u = 0; u < VU; ++u) {
-            const int idx = tid + 256 * u;
-            if (idx < DV * 16 * 8) *reinterpret_cast<uint4*>(Vs + (idx >> 3) * VR + (idx & 7) * 8) = vreg[u];
-        }
+        for (int u = 0; u < VU; ++u)
+            if (DV % 2 == 0 || tid + 256 * u < DV * 16 * 8) *reinterpret_cast<uint4*>(v_to + u * 32 * VR) = vreg[u];
     };
-    fetch_tiles(j_first);
-    for (int j0 = j_first; j0 <= block_last; j0 += 64) {
-        __syncthreads();                                                           // the previous tile is consumed
-        publish_tiles();
+    if (j_first + 64 * grp <= block_last) fetch_tiles(j_first + 64 * grp);
+    uint4 qf[DK];
+    {
+        const float* qr = p.q + (size_t)(first + (qvalid ? qi : 0)) * p.ldq + p.q_col0 + (size_t)h * p.dim;
+#pragma unroll
+        for (int kk = 0; kk < DK; ++kk) {
+            const int d = 32 * kk + 8 * kq;
+            float v[8];
+            if constexpr (VEC) {                                                         // (dim in whole 8s: a lane's 8 numbers are there or not)
+                const float4 x = seq_ld4(qr + (d < p.dim ? d : 0)), y = seq_ld4(qr + (d < p.dim ? d + 4 : 4));
+                v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w; v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = qr[d + i < p.dim ? d + i : 0];
+            }
+            uint32_t w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                w[i] = (qvalid && d + 2 * i < p.dim ? ZT<ZL_BF16>::from_f32(v[2 * i]) : 0) | (uint32_t)(qvalid && d + 2 * i + 1 < p.dim ? ZT<ZL_BF16>::from_f32(v[2 * i + 1]) : 0) << 16;
+            qf[kk] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    }
+    fa_f4 o[DV];
+#pragma unroll
+    for (int dt = 0; dt < DV; ++dt) o[dt] = (fa_f4){0.f, 0.f, 0.f, 0.f};
+    // scores, maximum and sink in powers of two
+    constexpr float kL2e = 1.4426950408889634f;
+    const float scale2 = p.scale * kL2e;
+    float m = p.sink && grp == 0 ? p.sink[h] * kL2e : -INFINITY, l = p.sink && grp == 0 ? 1.0f : 0.0f;
+
+    for (int jb = j_first; jb <= block_last; jb += 64 * NG) {
+        const int j0 = jb + 64 * grp;                                              // this group's tile
+        __syncthreads();                                                           // the previous tiles are consumed
+        if (j0 <= block_last) publish_tiles();
         __syncthreads();
-        if (j0 + 64 <= block_last) fetch_tiles(j0 + 64);                           // in flight during this tile's MFMAs
+        if (j0 + 64 * NG <= block_last) fetch_tiles(j0 + 64 * NG);                 // in flight during this tile's MFMAs
         if (j0 > wave_last) continue;                                              // wave-uniform; the barriers above stay in step
+        const bool whole = j0 + 63 <= wave_first && (p.window <= 0 || wave_last - j0 < p.window);      // every query of the wave sees every key
         fa_f4 sc[4];
         float mx = -INFINITY;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            sc[c] = (fa_f4){0.f, 0.f, 0.f, 0.f};
-            if (j0 + 16 * c <= wave_last) {
+        for (int c = 0; c < 4; ++c) sc[c] = (fa_f4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int kk = 0; kk < DK; ++kk) {
-                    const uint4 a = *reinterpret_cast<const uint4*>(Ks + (16 * c + nrow) * KR + 32 * kk + 8 * kq);
-                    sc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(fa_b8, a), __builtin_bit_cast(fa_b8, qf[kk]), sc[c], 0, 0, 0);
+        for (int kk = 0; kk < DK; ++kk)                                            // (four chains of products side by side)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const uint4 a = *reinterpret_cast<const uint4*>(Ks + (16 * c + nrow) * KR + 32 * kk + 8 * kq);
+                sc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(fa_b8, a), __builtin_bit_cast(fa_b8, qf[kk]), sc[c], 0, 0, 0);
+            }
+        if (whole) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                sc[c] *= scale2;
+                mx = fmaxf(fmaxf(fmaxf(mx, sc[c][0]), fmaxf(sc[c][1], sc[c][2])), sc[c][3]);
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int key = j0 + 16 * c + 4 * kq + r;
+                    const float v = (qvalid && key <= qpos && (p.window <= 0 || qpos - key < p.window)) ? sc[c][r] * scale2 : -INFINITY;
+                    sc[c][r] = v;
+                    mx = fmaxf(mx, v);
                 }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int key = j0 + 16 * c + 4 * kq + r;
-                const float v = (qvalid && key <= qpos && (p.window <= 0 || qpos - key < p.window)) ? sc[c][r] * p.scale : -INFINITY;
-                sc[c][r] = v;
-                mx = fmaxf(mx, v);
-            }
         }
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float mnew = fmaxf(m, mx);
-        const bool dead = mnew == -INFINITY;                                       // nothing seen yet and no sink: keep zeros
-        const float corr = dead ? 1.0f : __expf(m - mnew);
+        const float mnew = fmaxf(m, mx), mref = mnew == -INFINITY ? 0.f : mnew;    // (nothing seen yet and no sink: all weights are 2^-inf = 0)
+        const float corr = __builtin_amdgcn_exp2f(m - mref);
         float ps = 0.f;
         // the 32-key contraction of v_mfma_f32_16x16x32_bf16 may run over the keys in ANY order as long as both operands use the same one:
         // slot s of lane group kq stands for key 16 (s / 4) + 4 kq + s % 4 of the pair of 16-key blocks, which is how the scores lie here
@@ -615,15 +652,16 @@ __global__ __launch_bounds__(256) void k_latent_fa(const FaP p, const zls_batch_
         for (int c = 0; c < 4; ++c) {
 #pragma unroll
             for (int r = 0; r < 4; r += 2) {
-                uint16_t hb[2], lb[2];
+                uint32_t u[2], rest[2];
 #pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const float pv = (dead || sc[c][r + e] == -INFINITY) ? 0.f : __expf(sc[c][r + e] - mnew);
+                for (int e = 0; e < 2; ++e) {                                      // fa_split, two at a time
+                    const float pv = __builtin_amdgcn_exp2f(sc[c][r + e] - mref);
                     ps += pv;
-                    fa_split(pv, hb[e], lb[e]);
+                    u[e] = __builtin_bit_cast(uint32_t, pv);
+                    rest[e] = __builtin_bit_cast(uint32_t, pv - __builtin_bit_cast(float, u[e] & 0xffff0000u));
                 }
-                hi[c >> 1][2 * (c & 1) + (r >> 1)] = hb[0] | (uint32_t)hb[1] << 16;
-                lo[c >> 1][2 * (c & 1) + (r >> 1)] = lb[0] | (uint32_t)lb[1] << 16;
+                hi[c >> 1][2 * (c & 1) + (r >> 1)] = __builtin_amdgcn_perm(u[1], u[0], 0x07060302u);
+                lo[c >> 1][2 * (c & 1) + (r >> 1)] = __builtin_amdgcn_perm(rest[1], rest[0], 0x07060302u);
             }
         }
         ps += __shfl_xor(ps, 16, 64);
@@ -631,21 +669,46 @@ __global__ __launch_bounds__(256) void k_latent_fa(const FaP p, const zls_batch_
         l = l * corr + ps;
         m = mnew;
 #pragma unroll
-        for (int dt = 0; dt < DV; ++dt) {
-            o[dt] *= corr;
+        for (int dt = 0; dt < DV; ++dt) o[dt] *= corr;
 #pragma unroll
-            for (int c2 = 0; c2 < 2; ++c2) {
-                if (j0 + 32 * c2 <= wave_last) {                                    // (a block past the wave's last key has weights 0)
-                    const uint2 a0 = *reinterpret_cast<const uint2*>(Vs + (16 * dt + nrow) * VR + 32 * c2 + 4 * kq);
-                    const uint2 a1 = *reinterpret_cast<const uint2*>(Vs + (16 * dt + nrow) * VR + 32 * c2 + 16 + 4 * kq);
-                    const fa_b8 a = __builtin_bit_cast(fa_b8, make_uint4(a0.x, a0.y, a1.x, a1.y));
-                    const fa_b8 ph = __builtin_bit_cast(fa_b8, make_uint4(hi[c2][0], hi[c2][1], hi[c2][2], hi[c2][3]));
-                    const fa_b8 pl = __builtin_bit_cast(fa_b8, make_uint4(lo[c2][0], lo[c2][1], lo[c2][2], lo[c2][3]));
-                    o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ph, o[dt], 0, 0, 0);
-                    o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pl, o[dt], 0, 0, 0);
+        for (int c2 = 0; c2 < 2; ++c2) {                                           // (two outputs side by side)
+            const fa_b8 ph = __builtin_bit_cast(fa_b8, make_uint4(hi[c2][0], hi[c2][1], hi[c2][2], hi[c2][3]));
+            const fa_b8 pl = __builtin_bit_cast(fa_b8, make_uint4(lo[c2][0], lo[c2][1], lo[c2][2], lo[c2][3]));
+#pragma unroll
+            for (int d4 = 0; d4 < DV; d4 += 2) {
+                fa_b8 a[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const uint16_t* vr = Vs + (16 * (d4 + e) + nrow) * VR + 32 * c2 + 4 * kq;
+                    const uint2 a0 = *reinterpret_cast<const uint2*>(vr), a1 = *reinterpret_cast<const uint2*>(vr + 16);
+                    a[e] = __builtin_bit_cast(fa_b8, make_uint4(a0.x, a0.y, a1.x, a1.y));
                 }
+#pragma unroll
+                for (int e = 0; e < 2; ++e) o[d4 + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[e], ph, o[d4 + e], 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) o[d4 + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[e], pl, o[d4 + e], 0, 0, 0);
             }
         }
+    }
+    if constexpr (NG > 1) {                                                        // the second group hands its sums over, lane by lane
+        float* meet = reinterpret_cast<float*>(smem) + (size_t)wave * 64 * (DV * 4 + 2) + lane;
+        __syncthreads();
+        if (grp) {
+            meet[0] = m; meet[64] = l;
+#pragma unroll
+            for (int dt = 0; dt < DV; ++dt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) meet[64 * (2 + 4 * dt + r)] = o[dt][r];
+        }
+        __syncthreads();
+        if (grp) return;
+        const float m1 = meet[0], mm = fmaxf(m, m1), mref = mm == -INFINITY ? 0.f : mm;
+        const float f0 = __builtin_amdgcn_exp2f(m - mref), f1 = __builtin_amdgcn_exp2f(m1 - mref);
+        l = l * f0 + meet[64] * f1;
+#pragma unroll
+        for (int dt = 0; dt < DV; ++dt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[dt][r] = o[dt][r] * f0 + meet[64 * (2 + 4 * dt + r)] * f1;
     }
     if (!qvalid) return;
     const float g = p.gate ? seq_sigmoid(p.gate[(size_t)(first + qi) * p.ldg + p.g_col0 + h]) : 1.0f;
@@ -902,13 +965,18 @@ extern "C" int zls_latent_attention_prompt(const float* q, int64_t ldq, int64_t 
     p.ldq = ldq; p.ldg = ldg; p.ldk = ldk; p.ldv = ldv; p.q_col0 = (int)q_col0; p.g_col0 = (int)g_col0;
     p.heads = (int)heads; p.dim = (int)dim; p.vdim = (int)vdim; p.scale = scale; p.window = window > 0 ? (int)window : 0; p.ctx_pos0 = ctx_pos0;
     p.tiles_per_seq = (b->max_count + 63) / 64;
-    p.vec_k = (dim % 8 == 0 && ldk % 8 == 0 && ((uintptr_t)k & 15) == 0) ? 1 : 0;
-    const dim3 grid((unsigned)(b->n_seq * p.tiles_per_seq), (unsigned)heads);
+    const bool vec = dim % 8 == 0 && ldk % 8 == 0 && ldk < (1 << 24) && ldv < (1 << 24) && seq_aligned(k) && ldq % 4 == 0 && q_col0 % 4 == 0 && seq_aligned(q);
+    ZL_CHECK_ARG((int64_t)b->n_seq * p.tiles_per_seq * heads <= INT32_MAX, ZL_ELIMIT);
+    const dim3 grid((unsigned)(b->n_seq * p.tiles_per_seq * heads));
     hipStream_t hs = (hipStream_t)s;
+    // two groups where some query has more than four key tiles and the workgroups are few to a CU (two groups of long heads: 88 KB of LDS)
+    const bool pair = b->max_count > 128 && grid.x <= 1024;
     // the smallest instantiation that holds both the key size (32 DK) and the value size (16 DV): heads with a rotated part have keys
     // longer than their values
-#define FA(DK, DV) if (dim <= 32 * DK && vdim <= 16 * DV) { hipLaunchKernelGGL((k_latent_fa<DK, DV>), grid, dim3(256), 0, hs, p, *b); return zl_launch_status(); }
-    FA(1, 2) FA(2, 2) FA(2, 4) FA(4, 4) FA(4, 8) FA(6, 8) FA(8, 8) FA(8, 16)
+#define FA(DK, DV, NG, VEC) if (dim <= 32 * DK && vdim <= 16 * DV) { hipLaunchKernelGGL((k_latent_fa<DK, DV, NG, VEC>), grid, dim3(256 * NG), 0, hs, p, *b); return zl_launch_status(); }
+    if (vec && pair) { FA(2, 2, 2, true) FA(2, 4, 2, true) FA(4, 4, 2, true) FA(4, 8, 2, true) FA(6, 8, 2, true) }
+    if (vec) { FA(1, 2, 1, true) FA(2, 2, 1, true) FA(2, 4, 1, true) FA(4, 4, 1, true) FA(4, 8, 1, true) FA(6, 8, 1, true) FA(8, 8, 1, true) FA(8, 16, 1, true) }
+    FA(1, 2, 1, false) FA(2, 2, 1, false) FA(2, 4, 1, false) FA(4, 4, 1, false) FA(4, 8, 1, false) FA(6, 8, 1, false) FA(8, 8, 1, false) FA(8, 16, 1, false)
 #undef FA
     return ZL_ESHAPE;
 }

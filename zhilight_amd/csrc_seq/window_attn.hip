@@ -325,22 +325,26 @@ __global__ __launch_bounds__(256) void k_window_attention(const AttnP p, const z
 // Two P buffers alternate, so one barrier per page is enough.
 typedef __bf16 b8v __attribute__((ext_vector_type(8)));
 typedef float f4v __attribute__((ext_vector_type(4)));
-constexpr int kItems = 8;               // output blocks (16 value coordinates of one kv head) per wave: 4 waves x 8 x 16 = 512 per workgroup
+constexpr int kItems = 8;               // output blocks (16 value coordinates of one kv head) per wave, at most: 4 waves x 8 x 16 = 512 per workgroup
 
 __device__ __forceinline__ uint32_t bf16_bits(float f) {                 // round to nearest even; finite inputs
     uint32_t u = __builtin_bit_cast(uint32_t, f);
     u += 0x7fffu + ((u >> 16) & 1u);
     return u >> 16;
 }
-__device__ __forceinline__ void split8(const float* v, uint4& hi, uint4& lo) {
-    uint32_t h[8], l[8];
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef __bf16 b2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split8(const float* v, uint4& hi, uint4& lo) {      // hi = the nearest bf16 number, lo the nearest to the rest
+    uint32_t h[4], l[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        h[i] = bf16_bits(v[i]);
-        l[i] = bf16_bits(v[i] - __builtin_bit_cast(float, h[i] << 16));
+    for (int i = 0; i < 4; ++i) {
+        const f2v x = {v[2 * i], v[2 * i + 1]};
+        h[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, b2v));
+        const f2v rest = {x[0] - __builtin_bit_cast(float, h[i] << 16), x[1] - __builtin_bit_cast(float, h[i] & 0xffff0000u)};
+        l[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, b2v));
     }
-    hi = make_uint4(h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16);
-    lo = make_uint4(l[0] | l[1] << 16, l[2] | l[3] << 16, l[4] | l[5] << 16, l[6] | l[7] << 16);
+    hi = make_uint4(h[0], h[1], h[2], h[3]);
+    lo = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
 constexpr int kBiasLds = 2048;          // rows of a head's distance bias that the matrix-core kernel keeps in LDS (longer tables: the rest from memory)
@@ -351,15 +355,19 @@ __device__ __forceinline__ float fast_sigmoid(float x) {
 }
 __device__ __forceinline__ float fast_tanh(float x) { return 2.0f * fast_sigmoid(2.0f * x) - 1.0f; }
 
-template <int KS, int FORM>             // 32-coordinate steps of the head size: dim <= 32 KS; FORM 1: the general score form of AttnP with a
+// NI: output blocks of a wave (2 where that holds its share, or 8: blocks that are not there cost their products and registers all the same --
+// 16 heads of 128, 2952 tokens in a window of 1024: 215 us with 8, 115 with 2); up to 2 of them, the values of a page
+// are requested with its scores
+template <int KS, int FORM, int NI>     // 32-coordinate steps of the head size: dim <= 32 KS; FORM 1: the general score form of AttnP with a
                                         // softmax, 2: with sigmoid weights (no maximum, no correction of the sums, no normaliser),
                                         // 3: a softmax whose only addition is the linear distance bias (slope)
-__global__ __launch_bounds__(256) void k_window_attention_mfma(const AttnP p, const zls_batch_t b) {
+__global__ __launch_bounds__(256, KS <= 4 ? 2 : 1) void k_window_attention_mfma(const AttnP p, const zls_batch_t b) {
     __shared__ uint4 pfrag[2][4][2][2][64];                              // [buffer][query block][key half][hi, lo][lane]
     __shared__ float corr_s[2][64], l_s[64], m_s[64];
     __shared__ float bias_s[(FORM == 1 || FORM == 2) ? kBiasLds : 1];
-    const int tile = blockIdx.x, g = blockIdx.y, part = blockIdx.z;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nrow = lane & 15, kq = lane >> 4;
+    // (heads vary fastest and the tiles with the most keys behind them come first: the launch does not end on its longest workgroups)
+    const int tile = gridDim.x / p.heads - 1 - blockIdx.x / p.heads, g = blockIdx.x % p.heads, part = blockIdx.z;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nrow = lane & 15, kq = lane >> 4;
     const int t0 = p.tiles[3 * tile], rows = p.tiles[3 * tile + 1], sq = p.tiles[3 * tile + 2];
     const int pos0 = b.seq_pos0[sq] + (t0 - b.seq_start[sq]);
     const int G = p.kv_heads, d = p.dim, vd = p.vdim;
@@ -398,21 +406,21 @@ __global__ __launch_bounds__(256) void k_window_attention_mfma(const AttnP p, co
         __syncthreads();
     }
     uint4 qh[KS], ql[KS];
+    const float* qr = p.q + (size_t)(t0 + (qok ? qi : 0)) * p.ldq + p.q_col0 + g * d;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
         float v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int x = 32 * ks + 8 * kq + i;
-            v[i] = (qok && x < d) ? p.q[(size_t)(t0 + qi) * p.ldq + p.q_col0 + g * d + x] * qscale : 0.f;
-        }
+        for (int i = 0; i < 8; ++i) v[i] = qr[min(32 * ks + 8 * kq + i, d - 1)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = qok && 32 * ks + 8 * kq + i < d ? v[i] * qscale : 0.f;
         split8(v, qh[ks], ql[ks]);
     }
-    // this wave's output blocks: block index nb = (part * 4 * kItems) + wave + 4 i  ->  (kv head, 16 coordinates)
+    // this wave's output blocks: block index nb = (part * 4 * NI) + wave + 4 i  ->  (kv head, 16 coordinates)
     const int n_blocks = nv / 16, vb_per = vd / 16;
-    f4v acc[kItems][4];
+    f4v acc[NI][4];
 #pragma unroll
-    for (int i = 0; i < kItems; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
         for (int qb = 0; qb < 4; ++qb) acc[i][qb] = (f4v){0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
@@ -424,16 +432,32 @@ __global__ __launch_bounds__(256) void k_window_attention_mfma(const AttnP p, co
     // the key fragments of a page: A operands straight from the cache rows; the NEXT page's are requested as soon as this page's scores
     // are issued, and arrive during the softmax and the second product
     uint4 kf[4][KS];
+    uint32_t k_at[KS];                                                    // (numbers past the head: its last 8 again, the queries are 0 there)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) k_at[ks] = (uint32_t)nrow * (uint32_t)(G * d) + (uint32_t)min(32 * ks + 8 * kq, d - 8);
+    const uint32_t v_at = (uint32_t)nrow * 64 + 4 * kq;
     auto load_keys = [&](int pg) {
-        const size_t page = (size_t)pages[pg];
+        const uint16_t* base = kc + ((size_t)pages[pg] * 64 * G + c) * d;
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            const uint16_t* kr = kc + ((page * 64 + kb * 16 + nrow) * G + c) * d + 8 * kq;
+        for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-                kf[kb][ks] = (32 * ks + 8 * kq < d) ? *reinterpret_cast<const uint4*>(kr + 32 * ks) : make_uint4(0, 0, 0, 0);
+            for (int ks = 0; ks < KS; ++ks) kf[kb][ks] = *reinterpret_cast<const uint4*>(base + (size_t)(kb * 16) * G * d + k_at[ks]);
+    };
+    // the wave's V^T fragments of a key half, in the order of the P fragments
+    auto load_vals = [&](size_t page, int h2, uint4* vf) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int nb = part * 4 * NI + wave + 4 * i;
+            vf[i] = make_uint4(0, 0, 0, 0);
+            if (nb < n_blocks) {
+                const uint16_t* vr = vc + ((page * G + (p.all_kv ? nb / vb_per : c)) * vd + (nb % vb_per) * 16) * 64 + 32 * h2;
+                const uint2 a0 = *reinterpret_cast<const uint2*>(vr + v_at), a1 = *reinterpret_cast<const uint2*>(vr + v_at + 16);
+                vf[i] = make_uint4(a0.x, a0.y, a1.x, a1.y);
+            }
         }
     };
+    constexpr bool kEarly = NI <= 2;
+    uint4 ve[kEarly ? 2 : 1][NI];
     // the tile's pages: those that only hold kept first keys, then the pages from the oldest key any of its queries sees in its window
     const int wp0 = lo_key / 64, nkp = min((p.keep_first + 63) / 64, wp0), li_last = nkp + pg_last - wp0;
     auto page_of = [&](int li) { return li < nkp ? li : wp0 + li - nkp; };
@@ -441,21 +465,24 @@ __global__ __launch_bounds__(256) void k_window_attention_mfma(const AttnP p, co
     for (int li = 0; li <= li_last; ++li, buf ^= 1) {
         const int pg = page_of(li);
         const size_t page = (size_t)pages[pg];
+        if constexpr (kEarly) { load_vals(page, 0, ve[0]); load_vals(page, 1, ve[1]); }
         // ---- scores of the wave's 16 queries against the page's 64 keys
         f4v st[4];
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            st[kb] = (f4v){0.f, 0.f, 0.f, 0.f};
+        for (int kb = 0; kb < 4; ++kb) st[kb] = (f4v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                st[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, kf[kb][ks]), __builtin_bit_cast(b8v, qh[ks]), st[kb], 0, 0, 0);
-                st[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, kf[kb][ks]), __builtin_bit_cast(b8v, ql[ks]), st[kb], 0, 0, 0);
-            }
-        }
+        for (int ks = 0; ks < KS; ++ks)                                   // (four chains of products side by side)
+#pragma unroll
+            for (int hl = 0; hl < 2; ++hl)
+#pragma unroll
+                for (int kb = 0; kb < 4; ++kb)
+                    st[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, kf[kb][ks]), __builtin_bit_cast(b8v, hl ? ql[ks] : qh[ks]), st[kb], 0, 0, 0);
         if (li < li_last) load_keys(page_of(li + 1));
         // st[kb][r]: key pg * 64 + 16 kb + 4 kq + r, query nrow
         float cm = -INFINITY;
-        bool vis[4][4];
+        // every query of the wave sees every key of the page (rows past the tile see them too: nothing of theirs is kept)
+        const bool whole = (FORM == 0 || FORM == 3) && pg * 64 + 63 <= pos0 + 16 * wave && (p.window <= 0 || pos0 + 16 * wave + 15 - pg * 64 < p.window);
+        bool vis[4][4];                                                   // (not `whole`)
         float pw[4][4], psum = 0.f;
         if (FORM == 2) {
 #pragma unroll
@@ -472,26 +499,37 @@ __global__ __launch_bounds__(256) void k_window_attention_mfma(const AttnP p, co
                     pw[kb][r] = v ? __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(fmaf(sg_a, rr, bb))) : 0.f;
                 }
         }
+        if (FORM == 3) {
 #pragma unroll
-        for (int kb = 0; FORM != 2 && kb < 4; ++kb)
+            for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int j = pg * 64 + 16 * kb + 4 * kq + r;
-                vis[kb][r] = qok && j <= pq && (p.window <= 0 || pq - j < p.window || j < p.keep_first) && (FORM == 0 || FORM == 3 || j >= chunk0);
-                if (FORM == 3) st[kb][r] = fmaf(slope, (float)(j - pq), st[kb][r]);      // (the distance is an exact fp32 number)
-                if (FORM == 1 && vis[kb][r]) {
-                    float sv = st[kb][r];
-                    if (p.softcap > 0.f) sv = p.softcap * fast_tanh(sv * inv_cap);
-                    if (bias_lds) sv += bias_s[min(pq - j, p.bias_rows - 1)];
-                    else if (p.bias) {
-                        const int bi = min(pq - j, p.bias_rows - 1);
-                        sv += bi < kBiasLds ? bias_s[bi] : p.bias[(size_t)g * p.bias_rows + bi];
+                for (int r = 0; r < 4; ++r) st[kb][r] = fmaf(slope, (float)(pg * 64 + 16 * kb + 4 * kq + r - pq), st[kb][r]);      // (the distance is an exact fp32 number)
+        }
+        if (whole) {
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb) cm = fmaxf(fmaxf(fmaxf(cm, st[kb][0]), fmaxf(st[kb][1], st[kb][2])), st[kb][3]);
+        } else if (FORM != 2) {
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int j = pg * 64 + 16 * kb + 4 * kq + r;
+                    vis[kb][r] = (int)qok & (int)(j <= pq) & ((int)(p.window <= 0) | (int)(pq - j < p.window) | (int)(j < p.keep_first)) & (int)(FORM == 0 || FORM == 3 || j >= chunk0);
+                    if (FORM == 1 && vis[kb][r]) {
+                        float sv = st[kb][r];
+                        if (p.softcap > 0.f) sv = p.softcap * fast_tanh(sv * inv_cap);
+                        if (bias_lds) sv += bias_s[min(pq - j, p.bias_rows - 1)];
+                        else if (p.bias) {
+                            const int bi = min(pq - j, p.bias_rows - 1);
+                            sv += bi < kBiasLds ? bias_s[bi] : p.bias[(size_t)g * p.bias_rows + bi];
+                        }
+                        if (p.slope) sv = fmaf(slope, (float)(j - pq), sv);
+                        st[kb][r] = sv;
                     }
-                    if (p.slope) sv = fmaf(slope, (float)(j - pq), sv);
-                    st[kb][r] = sv;
+                    st[kb][r] = vis[kb][r] ? st[kb][r] : -INFINITY;
+                    cm = fmaxf(cm, st[kb][r]);
                 }
-                if (FORM != 2 && vis[kb][r]) cm = fmaxf(cm, st[kb][r]);
-            }
+        }
         constexpr bool sig = FORM == 2;
         if (!sig) {
             cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
@@ -501,11 +539,12 @@ __global__ __launch_bounds__(256) void k_window_attention_mfma(const AttnP p, co
         // (this kernel serves bf16 only: the hardware's exp2 is accurate to 1 ulp of the fp32 result, far inside what the bf16 keys leave)
         constexpr float kLog2e = 1.4426950408889634f;
         const float corr = (sig || m_new == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f((m_run - m_new) * kLog2e);
+        const float m_l2 = m_new == -INFINITY ? 0.f : m_new * kLog2e;     // (nothing seen yet: 2^-inf = 0)
 #pragma unroll
         for (int kb = 0; !sig && kb < 4; ++kb)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                pw[kb][r] = !vis[kb][r] ? 0.f : __builtin_amdgcn_exp2f((st[kb][r] - m_new) * kLog2e);
+                pw[kb][r] = __builtin_amdgcn_exp2f(fmaf(st[kb][r], kLog2e, -m_l2));
                 psum += pw[kb][r];
             }
         if (!sig) {
@@ -531,32 +570,25 @@ __global__ __launch_bounds__(256) void k_window_attention_mfma(const AttnP p, co
 #pragma unroll
             for (int qb = 0; qb < 4; ++qb) cq[qb] = corr_s[buf][16 * qb + nrow];
 #pragma unroll
-            for (int i = 0; i < kItems; ++i)
+            for (int i = 0; i < NI; ++i)
 #pragma unroll
                 for (int qb = 0; qb < 4; ++qb) acc[i][qb] *= cq[qb];
         }
 #pragma unroll
         for (int h2 = 0; h2 < 2; ++h2) {
-            uint4 vf[kItems];
-#pragma unroll
-            for (int i = 0; i < kItems; ++i) {
-                const int nb = part * 4 * kItems + wave + 4 * i;
-                vf[i] = make_uint4(0, 0, 0, 0);
-                if (nb < n_blocks) {
-                    const int cc = p.all_kv ? nb / vb_per : c, x = (nb % vb_per) * 16 + nrow;
-                    const uint16_t* vr = vc + ((page * G + cc) * vd + x) * 64 + 32 * h2 + 4 * kq;
-                    const uint2 a0 = *reinterpret_cast<const uint2*>(vr), a1 = *reinterpret_cast<const uint2*>(vr + 16);
-                    vf[i] = make_uint4(a0.x, a0.y, a1.x, a1.y);
-                }
-            }
+            uint4 late[NI];
+            if constexpr (!kEarly) load_vals(page, h2, late);
+            const uint4* vf = kEarly ? ve[kEarly ? h2 : 0] : late;
 #pragma unroll
             for (int qb = 0; qb < 4; ++qb) {
                 const uint4 bh = pfrag[buf][qb][h2][0][lane], bl = pfrag[buf][qb][h2][1][lane];
 #pragma unroll
-                for (int i = 0; i < kItems; ++i) {
+                for (int i = 0; i < NI; ++i) {
                     acc[i][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, vf[i]), __builtin_bit_cast(b8v, bh), acc[i][qb], 0, 0, 0);
-                    acc[i][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, vf[i]), __builtin_bit_cast(b8v, bl), acc[i][qb], 0, 0, 0);
                 }
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+                    acc[i][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, vf[i]), __builtin_bit_cast(b8v, bl), acc[i][qb], 0, 0, 0);
             }
         }
     }
@@ -571,8 +603,8 @@ __global__ __launch_bounds__(256) void k_window_attention_mfma(const AttnP p, co
         const float inv = 1.0f;
         float* out = p.acc + (((size_t)(t0 + row) * p.heads + g) * p.n_splits) * nv;
 #pragma unroll
-        for (int i = 0; i < kItems; ++i) {
-            const int nb = part * 4 * kItems + wave + 4 * i;
+        for (int i = 0; i < NI; ++i) {
+            const int nb = part * 4 * NI + wave + 4 * i;
             if (nb < n_blocks)
                 *reinterpret_cast<float4*>(out + nb * 16 + 4 * kq) = make_float4(acc[i][qb][0] * inv, acc[i][qb][1] * inv, acc[i][qb][2] * inv, acc[i][qb][3] * inv);
         }
@@ -825,15 +857,19 @@ extern "C" int zls_window_attention_prompt(const float* q, int64_t ldq, int64_t 
     if (st != ZL_OK) return st;
     const int64_t n_blocks = (all_kv ? kv_heads : 1) * vdim / 16, parts = (n_blocks + 4 * kItems - 1) / (4 * kItems);
     ZL_CHECK_ARG(parts <= 65535, ZL_ELIMIT);
-    const dim3 grid((unsigned)n_tiles, (unsigned)heads, (unsigned)parts);
+    ZL_CHECK_ARG(n_tiles * heads <= INT32_MAX, ZL_ELIMIT);
+    const dim3 grid((unsigned)(n_tiles * heads), 1, (unsigned)parts);
     hipStream_t hs = (hipStream_t)s;
     const int ks = (int)((dim + 31) / 32);
     const bool only_slope = form && form->slope && !form->head_scale && !(form->softcap > 0.f) && !form->bias && form->chunk == 0;
-#define PROMPT(KS)                                                                                      \
-    if (form && form->sigmoid) hipLaunchKernelGGL((k_window_attention_mfma<KS, 2>), grid, dim3(256), 0, hs, p, *b); \
-    else if (only_slope) hipLaunchKernelGGL((k_window_attention_mfma<KS, 3>), grid, dim3(256), 0, hs, p, *b); \
-    else if (form) hipLaunchKernelGGL((k_window_attention_mfma<KS, 1>), grid, dim3(256), 0, hs, p, *b); \
-    else hipLaunchKernelGGL((k_window_attention_mfma<KS, 0>), grid, dim3(256), 0, hs, p, *b)
+#define PROMPT_NI(KS, FORM)                                                                                                    \
+    if (n_blocks <= 8) hipLaunchKernelGGL((k_window_attention_mfma<KS, FORM, 2>), grid, dim3(256), 0, hs, p, *b);              \
+    else hipLaunchKernelGGL((k_window_attention_mfma<KS, FORM, kItems>), grid, dim3(256), 0, hs, p, *b)
+#define PROMPT(KS)                                            \
+    if (form && form->sigmoid) { PROMPT_NI(KS, 2); }          \
+    else if (only_slope) { PROMPT_NI(KS, 3); }                \
+    else if (form) { PROMPT_NI(KS, 1); }                      \
+    else { PROMPT_NI(KS, 0); }
     if (ks <= 1) { PROMPT(1); }
     else if (ks <= 2) { PROMPT(2); }
     else if (ks <= 3) { PROMPT(3); }
@@ -841,6 +877,7 @@ extern "C" int zls_window_attention_prompt(const float* q, int64_t ldq, int64_t 
     else if (ks <= 6) { PROMPT(6); }
     else { PROMPT(8); }
 #undef PROMPT
+#undef PROMPT_NI
     return zl_launch_status();
 }
 
