@@ -61,6 +61,8 @@ int zls_gemm_nt_act(const void* x, int64_t ldx, const void* w, const float* bias
  * x and w 16-byte aligned, otherwise ZL_ESHAPE. */
 int zls_gemm_nt_gated(const void* x, int64_t ldx, const void* w, const float* bias, int act, float alpha, float limit, void* y, int64_t ldy, int64_t m,
                       int64_t ff, int64_t k, zl_stream_t s);
+/* out row i = row rows[i] of x (device int32 indices); rows of row_bytes bytes in whole 16s, 16-byte aligned, otherwise ZL_ESHAPE */
+int zls_gather_rows(const void* x, const int32_t* rows, int64_t n_rows, int64_t row_bytes, void* out, zl_stream_t s);
 /* The same with gathered rows: row r of x is x[x_rows[r]], row c of w is w[w_rows[c]] (device int32 arrays, NULL: in order; ldw: row
  * stride of w).  Always the tiled kernel.  The up-projection of cached rows that lie scattered over pages. */
 int zls_gemm_nt_gather(const void* x, int64_t ldx, const int32_t* x_rows, const void* w, int64_t ldw, const int32_t* w_rows, void* y,

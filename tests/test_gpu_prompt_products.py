@@ -130,3 +130,11 @@ def test_int8_linear(m, n, k, dtype):
     add = torch.randn(m, n, device=DEV, generator=g).to(dtype)
     want = ops.quant_back_element_add_scale(c, sx, sy, add, 0.5)
     assert torch.equal(ops.int8_linear(a, sx, b, sy, addend=add, scale=0.5, out=add), want)
+
+
+@pytest.mark.parametrize("rows, width", [(1, 8), (64, 512), (131, 576), (300, 24)])
+def test_gathered_rows(rows, width):
+    from zhilight_amd import seqops
+    x = torch.randn(200, width, device=DEV).bfloat16()
+    at = torch.randint(0, 200, (rows,), device=DEV, dtype=torch.int32)
+    assert torch.equal(seqops.gather_rows(x, at), x[at.long()])

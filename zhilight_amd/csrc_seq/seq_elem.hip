@@ -574,6 +574,23 @@ __global__ __launch_bounds__(kT) void k_unary_act(const float* __restrict__ z, i
 
 }  // namespace
 
+// rows by index, 16 bytes a lane: 2048 rows of 512 bf16 numbers 4.4 us; the two products that read them run in 11.2 us each on rows in order, in 22.5
+// looking every row up
+static __global__ __launch_bounds__(256) void k_gather_rows(const uint4* __restrict__ x, const int32_t* __restrict__ rows, uint4* __restrict__ out, int64_t pieces, int per) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < pieces) out[i] = x[(size_t)rows[i / per] * per + i % per];
+}
+
+extern "C" int zls_gather_rows(const void* x, const int32_t* rows, int64_t n_rows, int64_t row_bytes, void* out, zl_stream_t s) {
+    ZL_CHECK_ARG(x && rows && out && n_rows > 0 && row_bytes > 0, ZL_EINVAL);
+    ZL_CHECK_ARG(row_bytes % 16 == 0 && row_bytes < (1 << 30) && seq_aligned(x) && seq_aligned(out), ZL_ESHAPE);
+    const int64_t pieces = n_rows * (row_bytes / 16);
+    ZL_CHECK_ARG((pieces + 255) / 256 <= INT32_MAX, ZL_ELIMIT);
+    hipLaunchKernelGGL(k_gather_rows, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, (hipStream_t)s, reinterpret_cast<const uint4*>(x), rows,
+                       reinterpret_cast<uint4*>(out), pieces, (int)(row_bytes / 16));
+    return zl_launch_status();
+}
+
 extern "C" int zls_embed(const int32_t* tokens, const void* table, const void* pos_table, int64_t vocab, int64_t max_positions, float scale,
                          const zls_batch_t* b, float* x, int64_t width, int dtype, zl_stream_t s) {
     ZL_CHECK_ARG(tokens && table && x && seq_batch_ok(b) && width > 0 && vocab > 0, ZL_EINVAL);

@@ -147,8 +147,13 @@ class LatentAttention(SideRows):
             flat = self.cache.view(-1, r)
             k = torch.empty((n_ctx, H * d), dtype=h.dtype, device=h.device)
             vt = torch.empty((H * self.vdim, n_ctx), dtype=h.dtype, device=h.device)
-            seqops.gemm_nt_gather(flat, ctx_rows, self.w_uk, None, n_ctx, H * d, k)
-            seqops.gemm_nt_gather(self.w_uv, None, flat, ctx_rows, H * self.vdim, n_ctx, vt)
+            if r % 64 == 0:                                                       # (rows that the large tiles take: brought together first)
+                rows = seqops.gather_rows(flat, ctx_rows)
+                seqops.gemm_nt(rows, self.w_uk, out=k)
+                seqops.gemm_nt(self.w_uv, rows, out=vt)
+            else:
+                seqops.gemm_nt_gather(flat, ctx_rows, self.w_uk, None, n_ctx, H * d, k)
+                seqops.gemm_nt_gather(self.w_uv, None, flat, ctx_rows, H * self.vdim, n_ctx, vt)
             seqops.latent_attention_prompt(proj, 0, gate, H * d + r, k, vt, self.sink, batch, self.scale, H, d, self.vdim, a, window=self.window)
         if not prompt or batch.n_single:
             seqops.latent_attention(proj, 0, gate, H * d + r, self.w_uk, self.w_uv, self.sink, self.cache, batch, self.scale, H, d, self.vdim,

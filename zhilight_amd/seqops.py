@@ -16,7 +16,7 @@ BF16, F32 = 1, 2
 _HERE = os.path.dirname(os.path.abspath(__file__))
 SO_PATH = os.path.join(_HERE, "libzhilight_amd_seq.so")
 SYMBOLS = ["zls_version", "zls_gemm_nt", "zls_gemm_nt_act", "zls_embed", "zls_token_shift", "zls_add_scalar_norm", "zls_scalar_norm_rows", "zls_polynorm",
-           "zls_latent_store", "zls_latent_attention", "zls_latent_attention_workspace_bytes", "zls_latent_attention_prompt", "zls_gemm_nt_gather",
+           "zls_latent_store", "zls_latent_attention", "zls_latent_attention_workspace_bytes", "zls_latent_attention_prompt", "zls_gemm_nt_gather", "zls_gather_rows",
            "zls_conv_silu", "zls_ssm_scan", "zls_ssm_scan_workspace_bytes", "zls_selective_scan", "zls_selective_scan_workspace_bytes", "zls_gated_group_norm", "zls_layer_norm",
            "zls_add_layer_norm", "zls_rope_norm_store", "zls_window_attention", "zls_window_attention_prompt", "zls_head_mix_gate", "zls_decay_scan", "zls_exp_gates",
            "zls_linear_attn_finish", "zls_moe_route", "zls_moe_align", "zls_gemm_nt_grouped", "zls_silu_mul", "zls_moe_combine", "zls_rms_norm",
@@ -341,8 +341,18 @@ def gemm_nt_gather(x, x_rows, w, w_rows, m, n, out):
     return out
 
 
+def gather_rows(x, rows):
+    """rows `rows` (int32, device) of a contiguous matrix whose rows come in whole 16 bytes"""
+    _cuda(x, rows)
+    if x.dim() != 2 or rows.dtype != torch.int32:
+        raise ZLError("gather_rows: a matrix and int32 row indices")
+    out = torch.empty((rows.numel(), x.shape[1]), dtype=x.dtype, device=x.device)
+    check(lib().zls_gather_rows(_p(x), _p(rows), _i(rows.numel()), _i(x.shape[1] * x.element_size()), _p(out), _stream()), "gather_rows")
+    return out
+
+
 def latent_attention_prompt(q, q_col0, gate, g_col0, k, vt, sink, batch, scale, heads, dim, vdim, out, window=0):
-    """the portions of the step on the matrix cores; k (n_ctx, heads * dim), vt (heads * vdim, n_ctx) from gemm_nt_gather over the rows of
+    """the portions of the step on the matrix cores; k (n_ctx, heads * dim), vt (heads * vdim, n_ctx) of the rows of
     batch.context(window); writes its rows of out"""
     _cuda(q, gate, k, vt, sink, out)
     _f32(q, gate, sink)
