@@ -168,3 +168,28 @@ def test_plain_heads_gate(heads, kv_heads, vdim, dtype):
             out = seqops.head_mix_gate(acc, ml, 1, None, None, None if kind is None else gate, col0, b, heads, kv_heads, vdim, dtype, sink=sk,
                                        plain_sum=plain, gate_per_head=kind == "head", out_scale=0.5)
             _close(out, ref, ref.abs(), 256)
+
+
+@pytest.mark.parametrize("bshd", [True, False])
+@pytest.mark.parametrize("tasks, len_q, hkv, d", [(1, 1, 1, 8), (3, 1, 8, 128), (1, 300, 36, 64), (2, 77, 3, 24), (1, 5, 40, 512), (2, 130, 1, 8)])
+def test_kv_scatter(tasks, len_q, hkv, d, bshd):
+    """whole numbers: every placed row where it belongs, slots below 0 and past the buffer never written"""
+    from zhilight_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(len_q + d)
+    k, v = (torch.randint(-9, 9, (tasks, len_q, hkv, d), device=DEV, generator=g).half() for _ in range(2))
+    lens = torch.tensor([len_q + 3 + i for i in range(tasks)], dtype=torch.int32, device=DEV)
+    place = torch.stack([torch.randperm(len_q + 5, device=DEV, generator=g)[:len_q] - 1 for _ in range(tasks)]).int()      # -1 .. len_q + 3
+    bufs = [[torch.full((n, hkv, d) if bshd else (hkv, n, d), 77.0, dtype=torch.float16, device=DEV) for n in lens.tolist()] for _ in range(2)]
+    want = [[x.clone() for x in side] for side in bufs]
+    for side, src in zip(want, (k, v)):
+        for b in range(tasks):
+            for t, p in enumerate(place[b].tolist()):
+                if 0 <= p < int(lens[b]):
+                    if bshd:
+                        side[b][p] = src[b, t]
+                    else:
+                        side[b][:, p] = src[b, t]
+    addr = [torch.tensor([x.data_ptr() for x in side], dtype=torch.int64, device=DEV) for side in bufs]
+    ops.copy_to_rag_buffer2(place.contiguous(), lens, k, v, *addr, bshd=bshd)
+    for side, ref in zip(bufs, want):
+        assert all(torch.equal(a, r) for a, r in zip(side, ref))
