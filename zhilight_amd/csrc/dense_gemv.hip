@@ -1,4 +1,4 @@
-// One row (and rows whose k is no whole 64s) runs k_dense_gemv, described next; 2 and more rows run zl_stream16.h.
+// One row (and rows whose k is no whole 64s) runs k_dense_gemv, described next; 2 and more rows run zl_stream16.h (the exceptions: at the dispatch).
 //
 // dense_gemv.hip -- y = T(alpha * x . W^T + bias) for small M (decode lm_head / NormalLinear), W (N,K)
 // fp16 or bf16 row-major.  SURVEY 8a row a21 (the reference calls cuBLASLt with fp32 compute:
@@ -302,8 +302,10 @@ static int gemm_nt_small_m_impl(const uint16_t* x, int64_t ldx, const uint16_t* 
     hipStream_t hs = (hipStream_t)s;
     // 2 and more rows: the streaming kernel; with a norm or a greedy pick up to 4 (x lies in LDS then).  One row: only narrow matrices, where its
     // shorter ramp counts (2304 x 5760 8.3 us against 9.6; 128256 x 4096 173 against 162) -- the norm and the pick stay with k_dense_gemv
-    const bool extra = norm_weight || argmax_ws;
-    if (s16_takes(x, ldx, w, m, n, k) && (m >= 2 ? !extra || (m <= 4 && (!norm_weight || k <= 8192)) : !extra && n <= 16384)) {
+    // Two fp16 rows of a wide matrix with a norm or a pick stay there too: its dot products take two numbers per instruction in fp16, and its loads leave
+    // no trace in the caches (2 x 128256 x 4096 inside a decode step: 165 us against 170, and 4 % less for the launches around it)
+    const bool extra = norm_weight || argmax_ws, two_halves = extra && m == 2 && n > 4096 && dtype == ZL_F16;
+    if (!two_halves && s16_takes(x, ldx, w, m, n, k) && (m >= 2 ? !extra || (m <= 4 && (!norm_weight || k <= 8192)) : !extra && n <= 16384)) {
         const Stream16P g = {x, w, ldx, (int)m, (int)n, (int)k, norm_weight, norm_eps, nullptr};
 #define ZL_STREAM(DT)                                                                                                                   \
     {                                                                                                                                   \

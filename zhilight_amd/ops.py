@@ -676,7 +676,7 @@ def gemm_nt(x, weight, bias=None, alpha=1.0, out=None):
 
 class DenseMWeight:
     """A dense (N, K) fp16 / bf16 matrix in the ZLD16M layout (zl_dense_pack_m): 16-row x 128-k tiles whose MFMA fragments are 1 KiB
-    contiguous -- for matrices streamed with 5..32 rows (the lm_head of a decode batch).  A second copy of the matrix: the row-major one
+    contiguous -- for matrices streamed with 9..32 rows (the lm_head of a decode batch).  A second copy of the matrix: the row-major one
     stays what the embedding, the 1..4-row GEMV and the prompt GEMM read."""
 
     def __init__(self, weight):
