@@ -372,7 +372,7 @@ class NormalLinear:
             x2 = ops.rmsnorm(x2, norm_weight, norm_eps)
         if ops.streams_rows(x2.shape[0], self.dim_out, self.dim_in):
             return ops.gemm_nt_small_m(x2, self.weight, bias=self.bias, out=out)
-        # 9..32 rows of a wide matrix (decode batches of the unquantised models, BASELINE configs[0]): the ZLD16M copy of the matrix -- 1 KiB contiguous
+        # 9..32 rows of a wide matrix (decode batches of the unquantised models): the ZLD16M copy of the matrix -- 1 KiB contiguous
         # fragment loads, 5.95 instead of 5.0 TB/s on the Llama-3 lm_head, the same bits; packed on first use outside stream capture.
         # A second copy of the weights: ZL_DENSE_PACKED=0 keeps only the row-major one
         if x2.shape[0] <= 32 and os.environ.get("ZL_DENSE_PACKED", "1") != "0":
